@@ -8,7 +8,8 @@
 //   codec_attention64   crates/omni-qwen3-tts/kernels/codec.cu:168-277
 //   dep_kv_attend64     crates/omni-personaplex/kernels/lm.cu:314-366
 //
-// One wave per (row, head). Lane l holds dims 8c .. 8c + 7 (c = l % 8, one
+// One wave per (row, head), eight per (rows of a session, head) for Mimi's
+// rings. Lane l holds dims 8c .. 8c + 7 (c = l % 8, one
 // 16-byte load of a 128-byte K or V row) of key row r = l / 8, so one load
 // instruction covers 8 keys; scores are 8-lane DPP sums and the softmax runs
 // online in base 2 with the scale folded into q. The key a fused kernel has
@@ -123,19 +124,6 @@ struct Row64 {
     l = fmaf(l, corr, ps);
   }
 
-  // Keys t = 0 .. len-1: K and V rows at kv.k(t), kv.v(t) (element pointers),
-  // 8 NI keys per round trip. (Two register tiles, the next one's loads in
-  // flight during this one's math, measured slower on Mimi's 250-key rings:
-  // 22.6 against 21.3 us per launch.)
-  template <int NI = 2, class KV>
-  __device__ void run(int len, const KV& kv, int cur, const uint4& cur_k, const uint4& cur_v) {
-    for (int tb = 0; tb < len; tb += 8 * NI) {
-      Tile<NI> x;
-      load(x, tb, len, kv);
-      step(x, tb, len, cur, cur_k, cur_v);
-    }
-  }
-
   // Sum the 8 key rows and write dims 8c .. 8c + 7 (lanes of key row 0).
   __device__ void finish(bf16_t* out) {
     const int lane = threadIdx.x & 63, c = lane & 7;
@@ -148,31 +136,134 @@ struct Row64 {
 };
 
 // ----------------------------------------------------------------- Mimi ring
-struct MimiRing {
-  const bf16_t* ring;
-  int first, context, heads, h;
-  __device__ const bf16_t* k(int t) const {
-    return ring + ((int64_t)((first + t) % context) * 2 * heads + h) * kD;
-  }
-  __device__ const bf16_t* v(int t) const {
-    return ring + ((int64_t)((first + t) % context) * 2 * heads + heads + h) * kD;
-  }
-};
+// Slots of one session's ring. A row at position p sees slots
+// (p - len + 1 + t) % context, t < len = min(p + 1, context): slots 0 .. len - 1
+// whether the ring has wrapped (all of them) or not, so the keys are walked in
+// slot order and the rows of one session see nested sets of slots.
+//
+// TR consecutive rows of one session (TR divides T) and one head per workgroup:
+// each K and V row is read once for the TR rows, and eight waves of two loads
+// of 8 slots each cover 128 slots per memory round trip (two for a full
+// 250-slot ring) where one wave per (row, head) walked it in sixteen. Bound by
+// those round trips in small batches and by memory in large ones. One frame of
+// eight layers at T = 2 with its codec and depformer calls, as a replayed
+// graph: 32 sessions 166 -> 79 us, 128 sessions 211 -> 152 us. Waves x loads
+// per trip, 4 / 32 / 128 sessions: 8 x 2 63 / 79 / 152, 4 x 4 66 / 83 / 150,
+// 8 x 4 61 / 80 / 180, 4 x 8 64 / 83 / 196 us (more loads per trip cost
+// registers, and so occupancy); one row per workgroup 58-60 / 91-95 / 199-209;
+// two heads per workgroup (256-byte runs) 71 / 85 / 153 us.
+constexpr int kMimiWaves = 8;
+constexpr int kMimiLoads = 2;
 
-__global__ __launch_bounds__(64) void mimi_attend64(ShortArgs a) {
-  const int n = blockIdx.x, h = blockIdx.y, c = threadIdx.x & 7;
-  const int s = n / a.T;
-  const int p = a.pos[s] * a.T + n % a.T;
-  const int len = min(p + 1, a.context);
-  float qv[8];
-  widen8(ldg16(a.qkv + ((int64_t)n * 3 * a.heads + h) * kD + 8 * c), qv);
-  Row64 st;
-  st.init(qv, a.scale);
-  const MimiRing ring{reinterpret_cast<const bf16_t*>(static_cast<const uint8_t*>(a.state) +
-                                                      (int64_t)a.lines[s] * a.stride),
-                      p - len + 1, a.context, a.heads, h};
-  st.run(len, ring, -1, uint4{}, uint4{});
-  st.finish(a.out + ((int64_t)n * a.heads + h) * kD);
+template <int TR>
+__global__ __launch_bounds__(64 * kMimiWaves) void mimi_attend64(ShortArgs a) {
+  constexpr int W = kMimiWaves, NI = kMimiLoads, R = 8;  // R slots per load instruction
+  const int n0 = blockIdx.x * TR, h = blockIdx.y;
+  const int lane = threadIdx.x & 63, c = lane & 7, r = lane >> 3;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int s = n0 / a.T;
+  const int p0 = a.pos[s] * a.T + n0 % a.T;
+  float q[TR][8], m[TR], l[TR], acc[TR][8];
+  int len[TR];
+#pragma unroll
+  for (int j = 0; j < TR; ++j) {
+    widen8(ldg16(a.qkv + ((int64_t)min(n0 + j, a.rows - 1) * 3 * a.heads + h) * kD + 8 * c), q[j]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      q[j][e] *= a.scale * kLog2e;
+      acc[j][e] = 0.f;
+    }
+    m[j] = -INFINITY;
+    l[j] = 0.f;
+    len[j] = min(p0 + j + 1, a.context);
+  }
+  const int64_t width = (int64_t)a.heads * kD;  // elements of a slot's K (and V) heads
+  const bf16_t* kb = reinterpret_cast<const bf16_t*>(static_cast<const uint8_t*>(a.state) +
+                                                     (int64_t)a.lines[s] * a.stride) + h * kD + 8 * c;
+  const int slots = len[TR - 1];
+  for (int tb = wave * R * NI; tb < slots; tb += W * R * NI) {
+    uint4 kr[NI], vr[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const bf16_t* at = kb + (int64_t)min(tb + R * i + r, slots - 1) * 2 * width;
+      kr[i] = ldg16_stream(at);
+      vr[i] = ldg16_stream(at + width);
+    }
+#pragma unroll
+    for (int j = TR - 1; j >= 0; --j) {
+      if (tb >= len[j]) continue;
+      // A slot that only a later row of the session sees: its p is 0 here, and
+      // its V row must not reach the sum (0 times an infinity would).
+      if (len[j] < slots) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+          if (tb + R * i + r >= len[j]) vr[i] = uint4{};
+      }
+      float sc[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        float kf[8];
+        widen8(kr[i], kf);
+        float d = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) d = fmaf(q[j][e], kf[e], d);
+        d = row8_sum64(d);
+        sc[i] = tb + R * i + r < len[j] ? d : -INFINITY;
+      }
+      float mx = sc[0];
+#pragma unroll
+      for (int i = 1; i < NI; ++i) mx = fmaxf(mx, sc[i]);
+      mx = across_rows8<true>(mx);
+      const float mn = fmaxf(m[j], mx);
+      const float corr = fast_exp2(m[j] - mn);
+      m[j] = mn;
+      float ps = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[j][e] *= corr;
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const float p = fast_exp2(sc[i] - mn);
+        ps += p;
+        float vf[8];
+        widen8(vr[i], vf);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[j][e] = fmaf(p, vf[e], acc[j][e]);
+      }
+      l[j] = fmaf(l[j], corr, ps);
+    }
+  }
+  // Merge the waves (a wave whose slots lie past the row's has m = -inf, l = 0).
+  __shared__ float sm_m[TR][W], sm_l[TR][W], sm_o[TR][W][kD];
+#pragma unroll
+  for (int j = 0; j < TR; ++j) {
+    l[j] = across_rows8<false>(l[j]);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[j][e] = across_rows8<false>(acc[j][e]);
+    if (r == 0) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sm_o[j][wave][8 * c + e] = acc[j][e];
+      if (c == 0) {
+        sm_m[j][wave] = m[j];
+        sm_l[j][wave] = l[j];
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < TR * kD; i += 64 * W) {
+    const int d = i % kD, j = i / kD;
+    if (n0 + j >= a.rows) break;
+    float top = sm_m[j][0];
+#pragma unroll
+    for (int w = 1; w < W; ++w) top = fmaxf(top, sm_m[j][w]);
+    float num = 0.f, den = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float e = sm_m[j][w] == -INFINITY ? 0.f : fast_exp2(sm_m[j][w] - top);
+      num = fmaf(sm_o[j][w][d], e, num);
+      den = fmaf(sm_l[j][w], e, den);
+    }
+    a.out[((int64_t)(n0 + j) * a.heads + h) * kD + d] = (bf16_t)f2bf(num / den);
+  }
 }
 
 // Mimi's rotary + ring write: row n of session s = n / T at p = pos[s] T +
@@ -316,7 +407,12 @@ int launch_short(const ShortArgs& a, int kind, hipStream_t stream) {
   if (a.rows == 0) return 0;
   const dim3 grid(a.rows, a.heads);
   switch (kind) {
-    case kShortMimi: mimi_attend64<<<grid, 64, 0, stream>>>(a); break;
+    case kShortMimi:  // an even T: a session's rows in pairs
+      if (a.T % 2 == 0)
+        mimi_attend64<2><<<dim3((a.rows + 1) / 2, a.heads), 64 * kMimiWaves, 0, stream>>>(a);
+      else
+        mimi_attend64<1><<<grid, 64 * kMimiWaves, 0, stream>>>(a);
+      break;
     case kShortCodec: codec_attention64<<<grid, 64, 0, stream>>>(a); break;
     case kShortDep: dep_kv_attend64<<<grid, 64, 0, stream>>>(a); break;
     case kShortMimiRope: mimi_rope_kv64<<<a.rows, 256, 0, stream>>>(a); break;

@@ -43,6 +43,37 @@ def test_mimi_attend(oracle, seed, context, pos_hi, sessions, T):
     assert_close(host_bits(out), want, what="mimi_attend")
 
 
+@pytest.mark.parametrize("T", [1, 2, 3, 4])
+@pytest.mark.parametrize("context", [8, 128, 260])
+def test_mimi_attend_rows_of_a_session(oracle, T, context):
+    """Ring lengths at the edges of a wave's and a workgroup's slots (16, 128),
+    every T a session's rows are taken by (pairs, single rows, an odd row
+    count), and infinite V in the slot that only a session's last row sees:
+    the other rows must not take it in. Tolerance as everywhere."""
+    at = np.array([0, 15, 16, 17, 127, 128, 129, 255, 256, 300])  # first row's position, before rounding to T
+    c = mimi_case(9, sessions=len(at), T=T, heads=3, context=context)
+    c["pos"] = (at // T).astype(np.int32)
+    slot = 2 * 3 * 64
+    rows = c["rows"] - (T == 2)  # a session cut short
+    keep = np.ones(rows, bool)
+    for i, p in enumerate(c["pos"]):
+        last = int(p) * T + T - 1
+        if T > 1 and last < context:
+            first = c["lines"][i] * c["stride"] // 2 + last * slot + slot // 2
+            c["state"].view(np.uint16)[first:first + slot // 2] = 0x7F80
+            keep[i * T + T - 1:(i + 1) * T] = False
+    args = (c["lines"], c["state"], c["rows"], T, 3, 0.125, context, c["stride"])
+    want = oracle.mimi_attend(c["qkv"], c["pos"], *args)
+    out = torch.zeros(c["rows"], 3 * 64, dtype=torch.bfloat16, device="cuda")
+    state = torch.from_numpy(c["state"]).cuda()
+    oa.mimi_attend(dev_bits(c["qkv"]), dev_i32(c["pos"]), dev_i32(c["lines"]), state, out, rows, T, 3, 0.125, context,
+                   c["stride"])
+    torch.cuda.synchronize()
+    got = host_bits(out)
+    assert not got[rows:].any()  # rows past the call's are not written
+    assert_close(got[:rows][keep], want[:rows][keep], what="mimi_attend")
+
+
 @pytest.mark.parametrize("seed,sessions,heads,pos_hi", [(4, 4, 4, 200), (5, 64, 16, 1000), (6, 3, 2, 3)])
 def test_codec_attention(oracle, seed, sessions, heads, pos_hi):
     c = codec_case(seed, sessions=sessions, heads=heads, pos_hi=pos_hi)
