@@ -14,6 +14,10 @@ import ctypes
 import os
 from dataclasses import dataclass
 
+# torch brings its own HIP runtime; it is loaded before the library so that the
+# library binds to the same one instead of pulling in a second copy from /opt/rocm.
+import torch as _torch
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libomni_attn.so")
 HEAD_DIM = 128
@@ -111,10 +115,6 @@ def load(path: str | None = None):
     path = path or os.environ.get("OMNI_ATTN_LIB") or LIB_PATH
     if not os.path.exists(path):
         raise OmniAttnError(ELAUNCH, f"{path} is missing: build it with pega-omni_amd/build.py")
-    # torch brings its own HIP runtime; load it first so the library binds to
-    # the same one instead of pulling in a second copy from /opt/rocm.
-    import torch  # noqa: F401
-
     L = ctypes.CDLL(path)
     P, i32, i64, f32 = ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_float
     dplan = ctypes.POINTER(DecodePlan)
@@ -176,33 +176,30 @@ def _check(rc: int):
         raise OmniAttnError(rc, load().omni_attn_last_error().decode())
 
 
+# A call's host time is most of a small launch's (4 sessions of one talker
+# layer: 13 us of host against 11 us of kernels), so the checks below read each
+# attribute once, pointers go to ctypes as plain integers (every pointer
+# parameter is declared c_void_p) and the stream is asked for as a raw handle
+# instead of a torch.cuda.Stream object.
 def _ptr(t):
-    if t is None:
-        return None
-    return ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
 def _stream(stream):
-    import torch
-
     if stream is None:
-        stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+        return _torch._C._cuda_getCurrentRawStream(_torch.cuda.current_device())
+    return stream.cuda_stream
 
 
 def _bf16_dev(t, name):
-    import torch
-
-    if t.dtype != torch.bfloat16 or not t.is_cuda or not t.is_contiguous():
+    if t.dtype != _torch.bfloat16 or not t.is_cuda or not t.is_contiguous():
         raise OmniAttnError(EINVAL, f"{name} must be a contiguous bf16 device tensor")
 
 
 def _i32_dev(t, name):
-    import torch
-
     if t is None:
         return
-    if t.dtype != torch.int32 or not t.is_cuda or not t.is_contiguous():
+    if t.dtype != _torch.int32 or not t.is_cuda or not t.is_contiguous():
         raise OmniAttnError(EINVAL, f"{name} must be a contiguous int32 device tensor")
 
 
@@ -210,15 +207,14 @@ def _ws(plan, workspace):
     """The workspace pointer for a decode run, after checking that it holds the
     plan's split partials (the C call takes no size: a smaller buffer would be
     written past its end)."""
-    need = int(plan.workspace_bytes)
     if workspace is None:
         return None
-    if workspace.numel() * workspace.element_size() < need:
-        raise OmniAttnError(EWORKSPACE, f"workspace holds {workspace.numel() * workspace.element_size()} bytes, "
-                                        f"the plan needs {need}")
+    need = plan.workspace_bytes
+    if workspace.nbytes < need:
+        raise OmniAttnError(EWORKSPACE, f"workspace holds {workspace.nbytes} bytes, the plan needs {need}")
     if not workspace.is_cuda or not workspace.is_contiguous():
         raise OmniAttnError(EINVAL, "workspace must be a contiguous device tensor")
-    return _ptr(workspace)
+    return workspace.data_ptr()
 
 
 # --------------------------------------------------------------------- decode
@@ -237,10 +233,8 @@ def decode_plan_fp8(rows: int, heads: int, page: int, max_len: int, chunk: int =
 
 def workspace_for(plan, device="cuda"):
     """Device workspace for a plan (None when the plan needs none)."""
-    import torch
-
     n = int(plan.workspace_bytes)
-    return torch.empty(n, dtype=torch.uint8, device=device) if n > 0 else None
+    return _torch.empty(n, dtype=_torch.uint8, device=device) if n > 0 else None
 
 
 def check_table(indptr_h, pages_h, num_pages, pos_h=None, seq_h=None, ragged=False, page=16, context=0):
@@ -300,10 +294,8 @@ def lm_attend_fp8(qkv, kv, pos, seq, ragged, indptr, pages, page, out, heads, sc
                   stream=None):
     """``lm_attend`` over FP8 E4M3 slots (crates/omni-personaplex/kernels/lm.cu:196-290).
     kv is a uint8 device tensor of slots of 2*heads*128 + 2*heads*4 bytes."""
-    import torch
-
     _bf16_dev(qkv, "qkv"), _bf16_dev(out, "out")
-    if kv.dtype != torch.uint8 or not kv.is_cuda or not kv.is_contiguous():
+    if kv.dtype != _torch.uint8 or not kv.is_cuda or not kv.is_contiguous():
         raise OmniAttnError(EINVAL, "kv must be a contiguous uint8 device tensor of FP8 slots")
     for t, n in ((pos, "pos"), (seq, "seq"), (indptr, "indptr"), (pages, "pages")):
         _i32_dev(t, n)
@@ -342,8 +334,6 @@ def prefill_plan(rows, hq, hk, page, seq_h, pos_h, device="cuda", exact_p=False)
     """Host plan of a ragged causal prefill; uploads the work list. exact_p:
     P carried as two bf16 terms through P.V (qwen3_attend's f32 P, ~1.4x the time)."""
     import numpy as np
-    import torch
-
     seq_a = np.ascontiguousarray(seq_h, dtype=np.int32)
     pos_a = np.ascontiguousarray(pos_h, dtype=np.int32)
     plan = PrefillPlan()
@@ -358,7 +348,7 @@ def prefill_plan(rows, hq, hk, page, seq_h, pos_h, device="cuda", exact_p=False)
                                          pos_a.ctypes.data_as(ctypes.c_void_p),
                                          work_h.ctypes.data_as(ctypes.c_void_p), cap, ctypes.byref(plan)))
     plan.exact_p = 1 if exact_p else 0
-    return Prefill(plan, torch.from_numpy(work_h).to(device))
+    return Prefill(plan, _torch.from_numpy(work_h).to(device))
 
 
 def prefill_run(pf: Prefill, qkv, kv, pos, seq, indptr, pages, out, scale, stream=None):
@@ -417,10 +407,9 @@ def lm_rope_attend_fp8(qkv, pos, slots, kv, indptr, pages, page, out, heads, coe
     """``lm_rope`` then ``lm_attend`` over FP8 slots (ragged = 0) in one launch:
     K and V of row n quantized into ``slots[n]`` (which must be the slot of ring
     index pos[n] % context), q rotated in registers only (qkv is not written)."""
-    import torch
     for t, n in ((qkv, "qkv"), (out, "out")):
         _bf16_dev(t, n)
-    if kv.dtype != torch.uint8 or not kv.is_cuda or not kv.is_contiguous():
+    if kv.dtype != _torch.uint8 or not kv.is_cuda or not kv.is_contiguous():
         raise OmniAttnError(EINVAL, "kv must be a contiguous uint8 device tensor of FP8 slots")
     for t, n in ((pos, "pos"), (slots, "slots"), (indptr, "indptr"), (pages, "pages")):
         _i32_dev(t, n)
@@ -441,10 +430,8 @@ def qwen3_rope_dense(qkv, q_norm, k_norm, kv, rows, per, base, span, hq, hk, eps
 def lm_rope(qkv, pos, slots, kv, rows, heads, coef, stream=None):
     """``lm_rope`` (crates/omni-personaplex/kernels/lm.cu:125-182): kv is a
     uint8 device tensor of FP8 slots."""
-    import torch
-
     _bf16_dev(qkv, "qkv"), _i32_dev(pos, "pos"), _i32_dev(slots, "slots")
-    if kv.dtype != torch.uint8 or not kv.is_cuda or not kv.is_contiguous():
+    if kv.dtype != _torch.uint8 or not kv.is_cuda or not kv.is_contiguous():
         raise OmniAttnError(EINVAL, "kv must be a contiguous uint8 device tensor of FP8 slots")
     _check(load().omni_lm_rope(_ptr(qkv), _ptr(pos), _ptr(slots), _ptr(kv), rows, heads, float(coef),
                                _stream(stream)))
@@ -515,9 +502,7 @@ def lm_dep_kv_attend(qkv, ws, step, out, rows, heads, scale, stream=None):
 
 def hidream_workspace(device="cuda"):
     """A workspace for hidream_attend_ws on the current device."""
-    import torch
-
-    return torch.empty(int(load().omni_hidream_workspace_bytes()), dtype=torch.uint8, device=device)
+    return _torch.empty(int(load().omni_hidream_workspace_bytes()), dtype=_torch.uint8, device=device)
 
 
 def hidream_attend_ws(q, k, v, out, q_len, kv_len_at, q_stride, causal, scale_log2, hq, hk, batch, q_bstride,
