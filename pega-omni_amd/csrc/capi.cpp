@@ -38,6 +38,14 @@ int ok() {
 
 hipStream_t as_stream(void* s) { return static_cast<hipStream_t>(s); }
 
+// Workgroups of the tiled kernel resident at once on the current device (one per CU).
+int resident_tiled_groups() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  return cus;
+}
+
 // Split size for a decode bucket: the largest chunk (<= 1024 keys) that
 // still gives the launch >= 4096 split workgroups at full length (16 per CU
 // on 256 CUs), down to 256. Measured on MI355X over seven bucket shapes: a
@@ -400,7 +408,8 @@ int omni_attn_prefill_run(const omni_attn_prefill_plan* plan, const void* qkv, c
   a.hk = plan->hk;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.exact_p = plan->exact_p;
-  const int rc = omni::launch_prefill(a, plan->workgroups, as_stream(stream));
+  a.subs = omni::tiled_subs(items, resident_tiled_groups());
+  const int rc = omni::launch_prefill(a, (int)items, as_stream(stream));
   if (rc == -2) return fail(OMNI_ATTN_EUNSUPPORTED, "prefill_run: shape not implemented");
   if (rc != 0) return fail(OMNI_ATTN_ELAUNCH, "prefill_run: launch failed: %s", hipGetErrorString(omni::g_launch_status));
   return ok();
@@ -420,14 +429,6 @@ int dit_alignment(const void* q, const void* k, const void* v, const void* out, 
     return fail(OMNI_ATTN_EINVAL, "hidream_attend: batch strides %lld / %lld / %lld are not multiples of 8 elements",
                 (long long)q_bstride, (long long)kv_bstride, (long long)out_bstride);
   return 0;
-}
-
-// Workgroups of the tiled kernel resident at once on the current device (one per CU).
-int resident_tiled_groups() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 0;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-  return cus;
 }
 
 }  // namespace
@@ -475,7 +476,12 @@ int dit_prepare(const void* q, const void* k, const void* v, void* out, int q_le
   return ok();
 }
 
-int dit_launch(const omni::TiledArgs& a, int batch, void* stream) {
+int dit_launch(omni::TiledArgs& a, int batch, void* stream) {
+  a.subs = 1;
+  if (a.split_k == 0 && a.halved == 0) {
+    const int per_tile = omni::kTiledRows / (a.hq / a.hk);
+    a.subs = omni::tiled_subs((long long)((a.q_len + per_tile - 1) / per_tile) * a.hk * batch, resident_tiled_groups());
+  }
   const int rc = omni::launch_dit(a, batch, as_stream(stream));
   if (rc == -2) return fail(OMNI_ATTN_EUNSUPPORTED, "hidream_attend: shape not implemented");
   if (rc != 0)

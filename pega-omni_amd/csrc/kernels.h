@@ -102,6 +102,8 @@ struct TiledArgs {
   int halved;
   // Prefill with P carried as two bf16 terms (hi + lo) through P.V.
   int exact_p;
+  // Workgroups per tile (1, 2 or 4; 2 and 4 only without split and halves).
+  int subs;
 };
 
 // Packed (position, head) query rows per MFMA tile: one 8-wave workgroup, one per CU.
@@ -114,7 +116,7 @@ constexpr int64_t kSegmentBytes = (int64_t)kTiledRows * (128 + 2) * 4;
 // (tile, kv head) item: sequence, first row, rows, kv head.
 constexpr int kPrefillWorkHeader = 16;
 constexpr int kXcds = 8;
-int launch_prefill(const TiledArgs& a, int workgroups, hipStream_t stream);
+int launch_prefill(const TiledArgs& a, int items, hipStream_t stream);
 
 // Rotary embedding + K/V scatter (the step before attention).
 struct RopeArgs {
@@ -156,6 +158,8 @@ int launch_rope(const RopeArgs& a, int mode, hipStream_t stream);
 int launch_dit(const TiledArgs& a, int batch, hipStream_t stream);
 // Items and the tail split launch_dit would use for a call (split_k = 0: none).
 void dit_split(const TiledArgs& a, int batch, int resident, int* items, int* split_from, int* split_k);
+// Workgroups per tile (TiledArgs::subs) for a call of `items` tiles.
+int tiled_subs(long long items, int resident);
 // Items launch_dit should run as row halves when no split is used (0: none).
 int dit_halves(const TiledArgs& a, int batch, int resident);
 

@@ -24,6 +24,7 @@
 //     LDS reads (ds_read_b64_tr_b16) per MFMA.
 // LDS layouts keep the MFMA operand reads conflict-free (see kTileElems).
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "kernels.h"
@@ -39,6 +40,7 @@ constexpr int kMB = kBN / 32;    // 32-key blocks per tile
 constexpr int kWaves = kTiledRows / 32;  // one 32-row query block per wave
 constexpr int kThreads = 64 * kWaves;
 constexpr int kRowsPerWave = kBN / kWaves;  // K/V tile rows each wave loads
+constexpr int kDmas = 2 * kRowsPerWave / 4;  // LDS DMAs a wave issues per tile: K rows, then V rows
 // LDS per buffer: the K tile then the V tile, each [128 keys][128] bf16 in
 // 256-byte rows, filled straight from global memory by LDS DMA
 // (buffer_load_dwordx4 ... lds for full tiles, global_load_lds_dwordx4 for the
@@ -131,23 +133,35 @@ struct Tile {
   int64_t per_slot;          // paged: elements per slot
 };
 
-template <int G, bool PAGED, bool HALVES = false, bool EXACT = false>
+// SUBS: workgroups per tile. 1: the eight waves own the tile's eight 32-row
+// blocks and each sees every key. 2 or 4: a workgroup takes 128 or 64 of the
+// tile's rows, waves w and w + 8 / SUBS own the same 32 rows, and each takes
+// its share (64 or 32 keys) of every 128-key tile; their partial (m, l, O)
+// merge in LDS at the end. For calls of too few tiles to fill the GPU.
+static_assert(kDmas == 8, "one DMA per K-step of the S stage");
+
+// Key sources: dense K and V; paged with pages that are multiples of the 16
+// rows a wave loads (a wave's rows of a tile lie in one page); any other page.
+constexpr int kDense = 0, kPagedWave = 1, kPagedLane = 2;
+
+template <int G, int SRC, int SUBS = 1, bool HALVES = false, bool EXACT = false>
 __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items, int ntiles) {
+  constexpr bool PAGED = SRC != kDense;
   // DiT, XCD-aware order: workgroup id i runs on XCD i % 8; give each XCD a
   // contiguous block of work items so the tiles sharing one K/V head (and
   // batch) share that XCD's L2.
   // Prefill: the work list gives each XCD a range of (tile, kv head) items,
   // ordered so the workgroups resident on an XCD share one (sequence, kv
   // head) and its K/V stays in that XCD's L2; workgroup i takes item
-  // start[i % 8] + i / 8 of its XCD's range.
+  // start[i % 8] + i / 8 (/ SUBS) of its XCD's range.
   // DiT tail split: the first split_from items run whole, then every later
   // item runs as split_k key chunks (workgroups dispatched after all whole
   // items, so they fill the last round), each with its own XCD-aware order.
   // DiT row halves (HALVES): the last `halved` items run as two workgroups
-  // of kBM / 2 packed rows, in the same order as the split chunks; waves
-  // 0..3 (one per SIMD) compute the first half, waves 4..7 the second, and
-  // all eight load the K/V tiles.
-  int idx, chunk = -1, half = -1;
+  // of kBM / 2 packed rows (as SUBS = 2), in the same order as the split
+  // chunks.
+  int idx, chunk = -1, sub = 0;
+  int subs = SUBS;  // workgroups this tile runs as
   if constexpr (HALVES) {
     const int halves_from = items - a.halved;
     const int whole8 = ((halves_from + 7) >> 3) << 3;
@@ -162,7 +176,8 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       const int u = (b2 & 7) * per + (b2 >> 3);
       if (u >= units) return;
       idx = halves_from + (u >> 1);
-      half = u & 1;
+      sub = u & 1;
+      subs = 2;
     }
   } else if (!PAGED && a.split_k > 0) {
     const int whole8 = ((a.split_from + 7) >> 3) << 3;
@@ -180,19 +195,26 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       chunk = u % a.split_k;
     }
   } else if (PAGED) {
-    const int x = blockIdx.x & 7;
-    idx = a.work[x] + (int)(blockIdx.x >> 3);
-    if (idx >= a.work[x + 1]) return;
+    // XCD x's range starts at header entry x, which the plan makes
+    // x (items / 8) + min(x, items % 8): computed, not read, so the item is
+    // the first load of the chain item -> sequence -> page ids -> K.
+    const int x = blockIdx.x & 7, k = blockIdx.x >> 3, j = k / SUBS;
+    if (j >= (items >> 3) + (x < (items & 7))) return;
+    idx = x * (items >> 3) + min(x, items & 7) + j;
+    sub = SUBS - 1 - k % SUBS;  // a tile's later rows see more keys
   } else {
-    const int per = (items + 7) >> 3;
-    idx = (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3));
-    if (idx >= items) return;
+    const int per = (items * SUBS + 7) >> 3;
+    const int u = (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3));
+    if (u >= items * SUBS) return;
+    idx = u / SUBS;
+    sub = SUBS - 1 - u % SUBS;
   }
   const int32_t* item = PAGED ? a.work + kPrefillWorkHeader + 4 * idx : nullptr;
   const int tile = PAGED ? 0 : idx % ntiles;
   const int kvh = PAGED ? item[3] : (idx / ntiles) % a.hk;
   const int b = PAGED ? 0 : idx / (ntiles * a.hk);
   constexpr int kPos = kBM / G;  // positions per tile
+  const int sub_pos = kPos / subs;  // positions of this workgroup: sub_pos * sub ..
 
   Tile t;
   if constexpr (PAGED) {
@@ -201,7 +223,8 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     t.pos = a.pos + first;
     t.q = a.q + (int64_t)first * a.q_stride;
     t.out = a.out + (int64_t)first * a.hq * kHead;
-    t.last = t.pos[t.nq - 1] + 1;
+    if (sub_pos * sub >= t.nq) return;  // a short tile: no rows here
+    t.last = t.pos[min(t.nq, sub_pos * (sub + 1)) - 1] + 1;
     t.len = t.last;
     t.pg = a.pages + a.indptr[s];
     t.per_slot = 2LL * a.hk * kHead;
@@ -214,10 +237,8 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     t.q = a.q + b * a.q_bstride + (int64_t)q0 * a.q_stride;
     t.out = a.out + b * a.out_bstride + (int64_t)q0 * a.hq * kHead;
     t.len = *a.kv_len_at;
-    // A half's rows end at position (kBM / 2) (half + 1) / G of the tile.
-    const int np = half < 0 ? t.nq : min(t.nq, (kBM / 2) * (half + 1) / G);
-    if (half > 0 && (kBM / 2) * half / G >= t.nq) return;  // a second half with no rows
-    t.last = a.causal ? min(t.len, q0 + np) : t.len;
+    if (sub_pos * sub >= t.nq) return;  // a short tile: no rows here
+    t.last = a.causal ? min(t.len, q0 + min(t.nq, sub_pos * (sub + 1))) : t.len;
     t.qpos0 = q0;
     t.kv_stride = (int64_t)a.hk * kHead;
     t.kbase = a.k + b * a.kv_bstride + (int64_t)kvh * kHead;
@@ -229,17 +250,24 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   __shared__ __align__(16) bf16_t smem0[kBufElems];
   __shared__ __align__(16) bf16_t smem1[kBufElems];
 
+  // Key tiles [s_lo, s_hi): all of them, or this chunk's share.
+  const int steps = (t.last + kBN - 1) / kBN;
+  const int s_lo = chunk < 0 ? 0 : chunk * steps / a.split_k;
+  const int s_hi = chunk < 0 ? steps : (chunk + 1) * steps / a.split_k;
+
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 31, h = lane >> 5;
 
-  // This lane's query column: packed row r = 32 wave + j.
-  const int r = wave * 32 + j;
-  const int p = r / G, head = kvh * G + r % G;
+  // This lane's query column: packed row r of the tile, in 32-row block rb.
+  // The wave's share of a key tile: its kg-th part of `subs`.
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  // Waves outside this workgroup's half, and waves none of whose 32 rows is a
-  // position of the tile (a short last tile), only load K/V tiles and meet
-  // the barriers (wave-uniform).
-  const bool active = (half < 0 || (wave_u >> 2) == half) && (32 * wave_u) / G < t.nq;
+  const int blocks = kWaves / subs;  // 32-row blocks of this workgroup
+  const int rb = blocks * sub + wave_u % blocks, kg = wave_u / blocks;
+  const int r = rb * 32 + j;
+  const int p = r / G, head = kvh * G + r % G;
+  // Waves none of whose 32 rows is a position of the tile (a short last
+  // tile) only load K/V tiles and meet the barriers (wave-uniform).
+  const bool active = (32 * rb) / G < t.nq;
   const bool row_ok = p < t.nq && active;
   int lim;  // keys this row sees
   if constexpr (PAGED)
@@ -257,9 +285,6 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       if (!row_ok) u = make_uint4(0, 0, 0, 0);
       qf[kk] = as_bf16x8(u);
     }
-    // Q is loaded once: wait for it here, so the key loop's first MFMA does
-    // not wait on the next tile's prefetch (vmcnt(0), other counters free).
-    __builtin_amdgcn_s_waitcnt(0x0F70);
   }
 
   // Loader: wave w fills rows kRowsPerWave w .. of the K and V tiles, four
@@ -269,11 +294,9 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   // Dense sources: within a full tile a lane's rows and chunks are fixed, so
   // its element offsets from the tile's first key are constants (32-bit) and a
   // tile adds one uniform base: loads take a scalar base and a vector offset.
-  // Paged sources with a page that is a multiple of kRowsPerWave: a wave's
-  // rows of a tile are consecutive keys of one page, so a tile needs one
-  // (scalar) page id per wave, read a tile ahead, and the rows are
-  // consecutive slots.
-  const bool page_wave = PAGED && a.pd.page % kRowsPerWave == 0;
+  // kPagedWave, pages that are multiples of kRowsPerWave: a wave's rows of a
+  // tile are consecutive keys of one page, so a tile needs one (scalar) page
+  // id per wave and the rows are consecutive slots.
   // Element offsets of this lane's rows from the first row of the wave's
   // block (dense: from the tile's first key): constants for every tile.
   uint32_t koff[kRowsPerWave / 4], voff[kRowsPerWave / 4];
@@ -291,70 +314,76 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       voff[i] = (uint32_t)(r0 * stride + 8 * vc);
     }
   }
-  // Page id of this wave's rows of the tile at key n (page_wave only).
-  // Loaded as a vector load a tile before use and made scalar only then, so
-  // reading it does not wait for the tile loads issued in between.
+  // Page ids of this wave's rows (kPagedWave): lane l holds the id of tile
+  // 64 b + l of the call's range, one vector load per 64 tiles, so issuing a
+  // tile costs a v_readlane and no wait that would drain the loads in flight.
   const __amdgpu_buffer_rsrc_t pg_rsrc =
       __builtin_amdgcn_make_buffer_rsrc(PAGED ? (void*)t.pg : nullptr, 0, -1, kBufferFlags);
-  auto wave_page = [&](int n) -> int {
-    const int i = page_index(a.pd, __builtin_amdgcn_readfirstlane(min(n + kRowsPerWave * wave_u, t.last - 1)));
-    return __builtin_amdgcn_raw_buffer_load_b32(pg_rsrc, 0, 4 * i, 0);
+  auto wave_pages = [&](int st) -> int {
+    const int64_t key = (int64_t)(st + lane) * kBN + kRowsPerWave * wave_u;
+    return __builtin_amdgcn_raw_buffer_load_b32(pg_rsrc, 4 * page_index(a.pd, (int)min(key, (int64_t)t.last - 1)), 0, 0);
   };
-  int next_pid = 0;  // page id for the next tile to issue (page_wave), per lane
-  auto issue_tile = [&](int n0, bf16_t* kd) {
-    bf16_t* vd = kd + kTileElems;
-    if (!PAGED || page_wave) {
-      // Rows past `last` (the key tile's tail) fall outside the buffer
-      // range and read as zeros: masked scores and zero V rows, so they add
-      // nothing, and no slot past the sequence's keys is read.
-      const bf16_t* kb;
-      const bf16_t* vb;
-      const int first = PAGED ? n0 + kRowsPerWave * wave_u : n0;  // key of this lane's row 0
-      const int rows = min(max(t.last - first, 0), PAGED ? kRowsPerWave : kBN);
-      const int64_t stride_bytes = 2 * (PAGED ? t.per_slot : t.kv_stride);
-      const int bytes = rows == (PAGED ? kRowsPerWave : kBN) ? -1 : (int)(rows * stride_bytes);
-      if constexpr (PAGED) {
-        const int64_t slot0 = page_slot(a.pd, __builtin_amdgcn_readfirstlane(next_pid), n0 + kRowsPerWave * wave_u);
-        kb = t.kbase + slot0 * t.per_slot;
-        vb = t.vbase + slot0 * t.per_slot;
-      } else {
-        kb = t.kbase + (int64_t)n0 * t.kv_stride;
-        vb = t.vbase + (int64_t)n0 * t.kv_stride;
+  int pids = 0;
+  // Buffer loads to LDS: the tile's base in a scalar resource, the lane's
+  // constant byte offsets in VGPRs, no per-lane address math. Rows past `last`
+  // (the key tile's tail) fall outside the buffer range and read as zeros:
+  // masked scores and zero V rows, so they add nothing, and no slot past the
+  // sequence's keys is read. A tile past the last is all such rows.
+  i32x4 k_rsrc, v_rsrc;
+  auto aim_tile = [&](int st) __attribute__((always_inline)) {
+    const int n0 = st * kBN;
+    const int first = PAGED ? n0 + kRowsPerWave * wave_u : n0;  // key of this lane's row 0
+    const int rows = st < s_hi ? min(max(t.last - first, 0), PAGED ? kRowsPerWave : kBN) : 0;
+    const int64_t stride_bytes = 2 * (PAGED ? t.per_slot : t.kv_stride);
+    const int bytes = rows == (PAGED ? kRowsPerWave : kBN) ? -1 : (int)(rows * stride_bytes);
+    int64_t off;
+    if constexpr (PAGED) {
+      const int at = st - s_lo;
+      if ((at & 63) == 0 && at > 0) pids = wave_pages(st);
+      off = page_slot(a.pd, __builtin_amdgcn_readlane(pids, at & 63), first) * t.per_slot;
+    } else {
+      off = (int64_t)n0 * t.kv_stride;
+    }
+    k_rsrc = buffer_rsrc(t.kbase + off, bytes);
+    v_rsrc = buffer_rsrc(t.vbase + off, bytes);
+  };
+  // DMA d of the aimed tile (K rows first, then V rows) into buffer kd.
+  auto dma_tile = [&](int d, bf16_t* kd) __attribute__((always_inline)) {
+    const int i = d % (kRowsPerWave / 4);
+    bf16_t* at = kd + (kRowsPerWave * wave_u + 4 * i) * kHead;
+    if (d < kRowsPerWave / 4)
+      dma_buffer16(k_rsrc, 2 * koff[i], at);
+    else
+      dma_buffer16(v_rsrc, 2 * voff[i], at + kTileElems);
+  };
+  // The whole tile st into buffer kd.
+  auto issue_tile = [&](int st, bf16_t* kd) __attribute__((always_inline)) {
+    if constexpr (SRC != kPagedLane) {
+      aim_tile(st);
+#pragma unroll
+      for (int d = 0; d < kDmas; ++d) dma_tile(d, kd);
+    } else {
+      // Any page size: offsets per lane first, then the loads (the offsets need
+      // the page ids); keys past `last` repeat the last key.
+      bf16_t* vd = kd + kTileElems;
+      int64_t koffs[kRowsPerWave / 4], voffs[kRowsPerWave / 4];
+#pragma unroll
+      for (int i = 0; i < kRowsPerWave / 4; ++i) {
+        const int row = kRowsPerWave * wave_u + 4 * i + (lane >> 4);
+        const int key = min(st * kBN + row, t.last - 1);
+        const int cs = lane & 15;
+        const int kc = cs ^ (row & 15);
+        const int vc = (((cs >> 2) ^ (row & 3)) << 2) | (cs & 3);
+        const int64_t off = page_slot(a.pd, t.pg[page_index(a.pd, key)], key) * t.per_slot;
+        koffs[i] = off + 8 * kc;
+        voffs[i] = off + 8 * vc;
       }
-      // Buffer loads to LDS: the tile's base in a scalar resource, the
-      // lane's constant byte offsets in VGPRs, no per-lane address math.
-      const i32x4 kr = buffer_rsrc(kb, bytes), vr = buffer_rsrc(vb, bytes);
 #pragma unroll
       for (int i = 0; i < kRowsPerWave / 4; ++i) {
         const int lrow = (kRowsPerWave * wave_u + 4 * i) * kHead;
-        dma_buffer16(kr, 2 * koff[i], kd + lrow);
-        dma_buffer16(vr, 2 * voff[i], vd + lrow);
+        dma_global16(t.kbase + koffs[i], kd + lrow);
+        dma_global16(t.vbase + voffs[i], vd + lrow);
       }
-      return;
-    }
-    // Offsets first, then the loads (the paged offsets need the page ids).
-    int64_t koffs[kRowsPerWave / 4], voffs[kRowsPerWave / 4];
-#pragma unroll
-    for (int i = 0; i < kRowsPerWave / 4; ++i) {
-      const int row = kRowsPerWave * wave_u + 4 * i + (lane >> 4);
-      const int key = min(n0 + row, t.last - 1);
-      const int cs = lane & 15;
-      const int kc = cs ^ (row & 15);
-      const int vc = (((cs >> 2) ^ (row & 3)) << 2) | (cs & 3);
-      int64_t off;
-      if constexpr (PAGED) {
-        off = page_slot(a.pd, t.pg[page_index(a.pd, key)], key) * t.per_slot;
-      } else {
-        off = (int64_t)key * t.kv_stride;
-      }
-      koffs[i] = off + 8 * kc;
-      voffs[i] = off + 8 * vc;
-    }
-#pragma unroll
-    for (int i = 0; i < kRowsPerWave / 4; ++i) {
-      const int lrow = (kRowsPerWave * wave_u + 4 * i) * kHead;
-      dma_global16(t.kbase + koffs[i], kd + lrow);
-      dma_global16(t.vbase + voffs[i], vd + lrow);
     }
   };
 
@@ -365,6 +394,7 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     for (int e = 0; e < 16; ++e) o[md][e] = 0.f;
   float m = -INFINITY, l = 0.f;
   const float sl2 = a.scale_log2;
+  const float grow_by = subs == 1 ? 8.f : 0.f;
 
   // Per-lane LDS bases (elements). S's A operand: K row 32 mb + j, chunk
   // 2 kk + h, in slot (2 kk + h) ^ (j & 15): elem = (k_lane ^ 16 kk) + 4096 mb.
@@ -378,35 +408,41 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   const int vg = lane >> 4, vi = lane & 15;
   const int v_lane = (4 * (vg >> 1) + (vi >> 2)) * kHead + 32 * (vi >> 2) + 16 * (vg & 1) + 4 * (vi & 3);
 
-  // Key tiles [s_lo, s_hi): all of them, or this chunk's share.
-  const int steps = (t.last + kBN - 1) / kBN;
-  const int s_lo = chunk < 0 ? 0 : chunk * steps / a.split_k;
-  const int s_hi = chunk < 0 ? steps : (chunk + 1) * steps / a.split_k;
-  if (page_wave && s_hi > s_lo) next_pid = wave_page(s_lo * kBN);
-  if (s_hi > s_lo) issue_tile(s_lo * kBN, smem0);
-  if (page_wave && s_lo + 1 < s_hi) next_pid = wave_page((s_lo + 1) * kBN);
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the first tile is in LDS
+  // The first tile. Q (and the page ids) were asked for above and are waited
+  // for with it, so the key loop's first MFMA does not wait on the next
+  // tile's loads.
+  if (SRC == kPagedWave && s_hi > s_lo) pids = wave_pages(s_lo);
+  if (s_hi > s_lo) issue_tile(s_lo, smem0);
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), other counters free
   __syncthreads();
-  // One key tile: start loading the next tile into `nxt`, compute from `cur`.
-  auto tile_step = [&](int st, const bf16_t* cur, bf16_t* nxt) {
-    const int n0 = st * kBN;
-    if (st + 1 < s_hi) issue_tile(n0 + kBN, nxt);  // lands while this tile computes
-    if (page_wave && st + 2 < s_hi) next_pid = wave_page(n0 + 2 * kBN);  // a tile ahead
-    const bf16_t* kt = cur;
-    const bf16_t* vt = cur + kTileElems;  // V tile
+  // One key tile: load the next tile into `nxt`, compute this wave's MB 32-key
+  // blocks of it (all four, or its share) from `cur`. The next tile's DMAs go
+  // out one per K-step of the S stage: issued together at the top of the step,
+  // the eight waves' 64 KiB kept the address unit busy and every wave waiting
+  // to issue for 0.45-0.75 us of a 3.1 us step, with the matrix cores idle.
+  auto tile_step = [&](auto mb_count, int st, const bf16_t* cur, bf16_t* nxt) __attribute__((always_inline)) {
+    constexpr int MB = decltype(mb_count)::value;
+    if constexpr (SRC != kPagedLane)
+      aim_tile(st + 1);
+    else if (st + 1 < s_hi)
+      issue_tile(st + 1, nxt);
+    const int own = MB == kMB ? 0 : 32 * MB * kg;  // the wave's first key of the tile
+    const int n0 = st * kBN + own;
+    const bf16_t* kt = cur + own * kHead;
+    const bf16_t* vt = cur + kTileElems + own * kHead;  // V tile
 
-    // S^T = K . Q^T for keys n0 .. n0 + kBN - 1: kMB interleaved MFMA chains
+    // S^T = K . Q^T for keys n0 .. n0 + 32 MB - 1: MB interleaved MFMA chains
     // (32-key blocks mb) over the 8 K-steps, with the K fragments read
     // from LDS two K-steps ahead of use; the stages are pinned in this order.
-    f32x16 sc[kMB];
+    f32x16 sc[MB];
 #pragma unroll
-    for (int mb = 0; mb < kMB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) sc[mb][e] = 0.f;
-    uint4 kf[8][kMB];
+    uint4 kf[8][MB];
     auto read_k = [&](int kk) {
 #pragma unroll
-      for (int mb = 0; mb < kMB; ++mb) kf[kk][mb] = *reinterpret_cast<const uint4*>(kt + (k_lane ^ (16 * kk)) + mb * 4096);
+      for (int mb = 0; mb < MB; ++mb) kf[kk][mb] = *reinterpret_cast<const uint4*>(kt + (k_lane ^ (16 * kk)) + mb * 4096);
     };
     read_k(0);
     read_k(1);
@@ -414,23 +450,24 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) {
 #pragma unroll
-      for (int mb = 0; mb < kMB; ++mb)
+      for (int mb = 0; mb < MB; ++mb)
         sc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[kk][mb]), qf[kk], sc[mb], 0, 0, 0);
+      if constexpr (SRC != kPagedLane) dma_tile(kk, nxt);
       if (kk + 2 < 8) read_k(kk + 2);
       __builtin_amdgcn_sched_barrier(0);
     }
 
     // Register e of block mb is key n0 + 32 mb + 8 (e / 4) + 4 h + e % 4.
-    if (__any(n0 + kBN > lim)) {
+    if (__any(n0 + 32 * MB > lim)) {
 #pragma unroll
-      for (int mb = 0; mb < kMB; ++mb)
+      for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
         for (int e = 0; e < 16; ++e)
           if (n0 + 32 * mb + 8 * (e >> 2) + 4 * h + (e & 3) >= lim) sc[mb][e] = -INFINITY;
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int mb = 0; mb < kMB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[mb][e]);
     {  // lanes l and l ^ 32 hold the two halves of the row's keys
@@ -439,9 +476,12 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     }
     // The running base m moves only when the max grows by more than 8 (log2):
     // p = 2^(s - m) <= 2^8 stays exact in f32 and l, O share the same base,
-    // so the result is unchanged while most tiles skip rescaling O.
+    // so the result is unchanged while most tiles skip rescaling O. A wave
+    // that sees only its share of a tile moves its base with every new max:
+    // its first tile holds a row's largest score less often, and p = 1 is the
+    // one value that rounding to bf16 leaves exact.
     const float mt = mx * sl2;
-    const bool grow = mt > m + 8.f;
+    const bool grow = mt > m + grow_by;
     if (__any(grow)) {
       const float alpha = grow ? fast_exp2(m - mt) : 1.f;
       m = grow ? mt : m;
@@ -454,7 +494,7 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     const float base = m == -INFINITY ? 0.f : m;
     float psum = 0.f;
 #pragma unroll
-    for (int mb = 0; mb < kMB; ++mb)
+    for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         sc[mb][e] = fast_exp2(fmaf(sc[mb][e], sl2, -base));
@@ -464,7 +504,7 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
 
     // O^T += V^T . P^T: K-step ks covers keys 16 ks + 4 h + {0..3, 8..11}.
 #pragma unroll
-    for (int ks_ = 0; ks_ < 2 * kMB; ++ks_) {
+    for (int ks_ = 0; ks_ < 2 * MB; ++ks_) {
       float pv[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) pv[e] = sc[ks_ >> 1][8 * (ks_ & 1) + e];
@@ -493,25 +533,28 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next tile has landed
     __syncthreads();
   };
-  // A wave that computes nothing: the same loads (its rows of every K/V
-  // tile, with the page ids a tile ahead) and barriers.
-  auto load_step = [&](int st, bf16_t* nxt) {
-    if (st + 1 < s_hi) issue_tile((st + 1) * kBN, nxt);
-    if (page_wave && st + 2 < s_hi) next_pid = wave_page((st + 2) * kBN);
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-  };
-  if (!active) {
-    for (int st = s_lo; st < s_hi; st += 2) {
-      load_step(st, smem1);
-      if (st + 1 < s_hi) load_step(st + 1, smem0);
+  if (!active) {  // computes nothing: the same loads (its rows of every K/V tile) and barriers
+    for (int st = s_lo; st < s_hi; ++st) {
+      if (st + 1 < s_hi) issue_tile(st + 1, (st - s_lo) & 1 ? smem0 : smem1);
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
+    }
+    if (SUBS > 1 || (HALVES && subs > 1)) {  // the merge's two
+      __syncthreads();
+      __syncthreads();
     }
     return;
   }
-  for (int st = s_lo; st < s_hi; st += 2) {
-    tile_step(st, smem0, smem1);
-    if (st + 1 < s_hi) tile_step(st + 1, smem1, smem0);
-  }
+  auto key_loop = [&](auto mb_count) __attribute__((always_inline)) {
+    for (int st = s_lo; st < s_hi; st += 2) {  // unrolled by two: buffer addresses are constants
+      tile_step(mb_count, st, smem0, smem1);
+      if (st + 1 < s_hi) tile_step(mb_count, st + 1, smem1, smem0);
+    }
+  };
+  if (HALVES && subs > 1)
+    key_loop(std::integral_constant<int, kMB / 2>{});
+  else
+    key_loop(std::integral_constant<int, kMB / SUBS>{});
 
   // Register e of block md is dim 32 md + 8 (e / 4) + 4 h + e % 4.
   l += xor_lane(l, 32);
@@ -527,21 +570,83 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     if (h == 0) *reinterpret_cast<float2*>(seg + kBM * kHead + 2 * r) = make_float2(m, l);
     return;
   }
-  // Normalise and store. A row that sees no key (*kv_len_at = 0) has l = 0 and
-  // O = 0, and stores 0 * (1 / 0) = NaN, as hidream.cu:333-346 does.
-  if (!row_ok) return;
-  const float inv = 1.f / l;
-  bf16_t* dst = t.out + ((int64_t)p * a.hq + head) * kHead;
+  // Waves that share rows exchange their partials through the (now free) tile
+  // buffers: 16 KiB of O per wave, element (md, q4) of lane l at 16-byte slot
+  // 64 (4 md + q4) + l. Wave kg of a row block then merges and stores the
+  // dims of blocks md = kg * 4 / subs .. + 4 / subs - 1.
+  int md_lo = 0, md_n = 4;
+  if constexpr (SUBS > 1 || HALVES) {
+    if (subs > 1) {
+      __shared__ float2 s_ml[kWaves][64];
+      auto region = [&](int w) { return reinterpret_cast<float4*>(w < 4 ? smem0 : smem1) + (w & 3) * 1024; };
 #pragma unroll
-  for (int md = 0; md < 4; ++md)
+      for (int md = 0; md < 4; ++md)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+          region(wave_u)[64 * (4 * md + q4) + lane] =
+              make_float4(o[md][4 * q4], o[md][4 * q4 + 1], o[md][4 * q4 + 2], o[md][4 * q4 + 3]);
+      s_ml[wave][lane] = make_float2(m, l);
+      __syncthreads();
+      md_n = 4 / subs;
+      md_lo = kg * md_n;
+      float top = -INFINITY;
+      for (int g = 0; g < subs; ++g) top = fmaxf(top, s_ml[wave_u % blocks + g * blocks][lane].x);
+#pragma unroll
+      for (int md = 0; md < 4 / (SUBS > 1 ? SUBS : 2); ++md)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[md][e] = 0.f;
+      l = 0.f;
+      for (int g = 0; g < subs; ++g) {
+        const int w = wave_u % blocks + g * blocks;
+        const float2 ml = s_ml[w][lane];
+        const float f = ml.x == -INFINITY ? 0.f : fast_exp2(ml.x - top);
+        l = fmaf(ml.y, f, l);
+#pragma unroll
+        for (int md = 0; md < 4 / (SUBS > 1 ? SUBS : 2); ++md)
+#pragma unroll
+          for (int q4 = 0; q4 < 4; ++q4) {
+            const float4 v = region(w)[64 * (4 * (md_lo + md) + q4) + lane];
+            o[md][4 * q4 + 0] = fmaf(v.x, f, o[md][4 * q4 + 0]);
+            o[md][4 * q4 + 1] = fmaf(v.y, f, o[md][4 * q4 + 1]);
+            o[md][4 * q4 + 2] = fmaf(v.z, f, o[md][4 * q4 + 2]);
+            o[md][4 * q4 + 3] = fmaf(v.w, f, o[md][4 * q4 + 3]);
+          }
+      }
+    }
+  }
+  // Normalise and store. A row that sees no key (*kv_len_at = 0) has l = 0 and
+  // O = 0, and stores 0 * (1 / 0) = NaN, as hidream.cu:333-346 does. The rows
+  // go through LDS (64 (d / 8) + lane order undone by the read) so that a
+  // store instruction writes whole contiguous runs of a row instead of 8
+  // bytes of 32 different rows: 16-byte chunk c of block row j sits in slot
+  // c ^ (j & 15) of its row, and the wave alone uses its 8 KiB.
+  const float inv = 1.f / l;
+  constexpr int kDims = kHead / SUBS;  // dims this wave stores (half of them in the halves' workgroups)
+  if constexpr (SUBS > 1 || HALVES)
+    if (subs > 1) __syncthreads();  // the merge's reads are over
+  bf16_t* rows = (wave_u < 4 ? smem0 : smem1) + (wave_u & 3) * 32 * kHead;
+#pragma unroll
+  for (int md = 0; md < 4 / SUBS; ++md)
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
-      const int d = 32 * md + 8 * q4 + 4 * h;
+      if (HALVES && md >= md_n) break;
+      // dims 32 md + 8 q4 + 4 h .. + 3 of this wave's: half h of chunk 4 md + q4
       uint2 w;
       w.x = pack_bf16x2(o[md][4 * q4 + 0] * inv, o[md][4 * q4 + 1] * inv);
       w.y = pack_bf16x2(o[md][4 * q4 + 2] * inv, o[md][4 * q4 + 3] * inv);
-      *reinterpret_cast<uint2*>(dst + d) = w;
+      *reinterpret_cast<uint2*>(rows + j * kHead + 8 * ((4 * md + q4) ^ (j & 15)) + 4 * h) = w;
     }
+  // The block's rows, 16-byte chunk by chunk: the wave's own LDS writes, in order.
+  const int chunks = HALVES ? 4 * md_n : kDims / 8;  // 16-byte chunks of a row
+#pragma unroll
+  for (int i = 0; i < 8 / SUBS; ++i) {
+    if (HALVES && i >= 2 * md_n) break;
+    const int at = 64 * i + lane, jr = at / chunks, c = at % chunks;
+    const int rr = rb * 32 + jr, pr = rr / G;
+    const uint4 w = *reinterpret_cast<const uint4*>(rows + jr * kHead + 8 * (c ^ (jr & 15)));
+    if (pr < t.nq)
+      *reinterpret_cast<uint4*>(t.out + ((int64_t)pr * a.hq + kvh * G + rr % G) * kHead + 32 * md_lo + 8 * c) = w;
+  }
 }
 
 // Merge the split_k chunk partials of each split DiT item into its output
@@ -611,23 +716,35 @@ __global__ __launch_bounds__(256) void dit_combine(TiledArgs a, int ntiles) {
   *reinterpret_cast<uint4*>(a.out + b * a.out_bstride + ((int64_t)(q0 + p) * a.hq + head) * kHead + d0) = o;
 }
 
-// Prefill with exact_p set: the hi + lo P.V variant (prefill only; DiT rounds
-// P to bf16 as hidream.cu does). Returns whether it launched.
-template <int G, bool PAGED>
-bool launch_exact(const TiledArgs& a, int grid, int items, int ntiles, hipStream_t stream) {
-  if constexpr (PAGED) {
-    if (a.exact_p) {
-      tiled_attn<G, true, false, true><<<grid, kThreads, 0, stream>>>(a, items, ntiles);
-      return true;
-    }
-  }
-  return false;
+template <int G, int SRC, int SUBS>
+void launch_subs(const TiledArgs& a, int grid, int items, int ntiles, hipStream_t stream) {
+  // Prefill with exact_p set: the hi + lo P.V variant (prefill only; DiT
+  // rounds P to bf16 as hidream.cu does).
+  if (SRC != kDense && a.exact_p)
+    tiled_attn<G, SRC, SUBS, false, SRC != kDense><<<grid, kThreads, 0, stream>>>(a, items, ntiles);
+  else
+    tiled_attn<G, SRC, SUBS><<<grid, kThreads, 0, stream>>>(a, items, ntiles);
+}
+
+template <int G, int SRC>
+void launch_g(const TiledArgs& a, int grid, int items, int ntiles, hipStream_t stream) {
+  if (a.subs == 4)
+    launch_subs<G, SRC, 4>(a, grid, items, ntiles, stream);
+  else if (a.subs == 2)
+    launch_subs<G, SRC, 2>(a, grid, items, ntiles, stream);
+  else
+    launch_subs<G, SRC, 1>(a, grid, items, ntiles, stream);
 }
 
 template <bool PAGED>
-int launch_tiled(const TiledArgs& a, int items, int ntiles, hipStream_t stream) {
+int launch_tiled(const TiledArgs& args, int items, int ntiles, hipStream_t stream) {
   if (items <= 0) return 0;
-  int grid = ((items + 7) >> 3) << 3;
+  TiledArgs a = args;
+  // Pages that are no multiple of a wave's rows keep one workgroup per tile.
+  const bool lane_pages = PAGED && a.pd.page % kRowsPerWave != 0;
+  if (lane_pages) a.subs = 1;
+  // Prefill: the XCDs' item ranges differ by one, each item `subs` workgroups.
+  int grid = PAGED ? (((items + 7) >> 3) << 3) * a.subs : ((items * a.subs + 7) >> 3) << 3;
   if (!PAGED && a.split_k > 0)
     grid = (((a.split_from + 7) >> 3) << 3) + ((((items - a.split_from) * a.split_k + 7) >> 3) << 3);
   const bool halves = !PAGED && a.split_k == 0 && a.halved > 0;
@@ -636,9 +753,11 @@ int launch_tiled(const TiledArgs& a, int items, int ntiles, hipStream_t stream) 
 #define OMNI_CASE(G)                                                                       \
   case G:                                                                                  \
     if (halves)                                                                            \
-      tiled_attn<G, false, true><<<grid, kThreads, 0, stream>>>(a, items, ntiles);         \
-    else if (!launch_exact<G, PAGED>(a, grid, items, ntiles, stream))                      \
-      tiled_attn<G, PAGED><<<grid, kThreads, 0, stream>>>(a, items, ntiles);               \
+      tiled_attn<G, kDense, 1, true><<<grid, kThreads, 0, stream>>>(a, items, ntiles);     \
+    else if (lane_pages)                                                                   \
+      launch_subs<G, PAGED ? kPagedLane : kDense, 1>(a, grid, items, ntiles, stream);      \
+    else                                                                                   \
+      launch_g<G, PAGED ? kPagedWave : kDense>(a, grid, items, ntiles, stream);            \
     break;
     OMNI_CASE(1)
     OMNI_CASE(2)
@@ -655,8 +774,8 @@ int launch_tiled(const TiledArgs& a, int items, int ntiles, hipStream_t stream) 
   return 0;
 }
 
-int launch_prefill(const TiledArgs& a, int workgroups, hipStream_t stream) {
-  return launch_tiled<true>(a, workgroups, 0, stream);
+int launch_prefill(const TiledArgs& a, int items, hipStream_t stream) {
+  return launch_tiled<true>(a, items, 0, stream);
 }
 
 int launch_dit(const TiledArgs& a, int batch, hipStream_t stream) {
@@ -669,15 +788,26 @@ int launch_dit(const TiledArgs& a, int batch, hipStream_t stream) {
   return launch_tiled<false>(a, (int)items, ntiles, stream);
 }
 
+// Workgroups per tile for a call of `items` tiles on `resident` CUs: as many as
+// still fit one round. A workgroup of a half (quarter) of a tile's rows takes
+// 0.68 (0.4-0.5) of a whole one's time, so a second round would lose what the
+// split wins. us per launch, replayed graph, 1 / 2 / 4 workgroups per tile:
+// 187 rows of 16q/8kv (16 tiles) 10.3 / 10.9 / 9.5; three requests of 60-400
+// rows over 700-3100 cached keys, 32q/8kv, exact P (104 tiles) 89 / 61 / 68;
+// 1025 DiT rows over 1102 keys (136 tiles, two rounds when split) 33 / 45 / 50.
+int tiled_subs(long long items, int resident) {
+  if (items * 4 <= resident) return 4;
+  return items * 2 <= resident ? 2 : 1;
+}
+
 // Without a workspace: when the last round holds at most half the resident
 // workgroups, its items run as row halves (two workgroups each, on twice the
-// CUs); with one computing wave per SIMD such a round takes about 0.7 of a
-// full round's time.
+// CUs); such a round takes about 0.7 of a full round's time.
 int dit_halves(const TiledArgs& a, int batch, int resident) {
   const int G = a.hq / a.hk;
   const int ntiles = (a.q_len + kBM / G - 1) / (kBM / G);
   const long long n = (long long)ntiles * a.hk * batch;
-  if (resident <= 0 || n <= 0 || n > (1LL << 30)) return 0;
+  if (resident <= 0 || n < resident || n > (1LL << 30)) return 0;  // less than a round: tiled_subs
   const int rem = (int)(n % resident);
   return 2 * rem > resident ? 0 : rem;
 }
@@ -698,7 +828,12 @@ void dit_split(const TiledArgs& a, int batch, int resident, int* items, int* spl
   *items = (int)n;
   *split_from = (int)n;
   *split_k = 0;
-  if (resident <= 0 || n <= 0 || n > (1LL << 30)) return;
+  // Calls of less than one round split their tiles by rows within the launch
+  // instead (tiled_subs): no partials in memory and no combine launch. 32q/8kv,
+  // us per call, by keys / by rows: 65 queries x 142 keys 17.2 / 11.6, 257 x 334
+  // 22.6 / 13.6, 1000 x 1077 37.8 / 27.5; key splits would win only for few
+  // queries over many keys (257 x 4096 56 / 61), which DiT calls are not.
+  if (resident <= 0 || n < resident || n > (1LL << 30)) return;
   const int rem = (int)(n % resident);
   if (rem == 0 || resident / rem < 2) return;
   const int chunks = std::min(resident / rem, std::max(2, (a.q_len + kBN - 1) / kBN / kMinChunkTiles));

@@ -329,6 +329,62 @@ def test_prefill_long_sequence(oracle):
     assert_close(got[pick], oracle_paged(oracle, sub), what="long prefill, first and last rows")
 
 
+@pytest.mark.parametrize("exact_p", [False, True])
+@pytest.mark.parametrize("rows,cached,hq,hk", [
+    # with 256 CUs: 64 (tile, kv head) items or fewer run as four workgroups per
+    # tile, 128 or fewer as two, more as one
+    (16, 0, 32, 8), (17, 200, 32, 8), (513, 5, 32, 8),  # four: a quarter tile, one row more, 72 items -> two
+    (512, 31, 16, 8), (1024, 0, 16, 8), (2048, 127, 16, 8), (2049, 0, 16, 8),  # 32, 64 (four), 128 (two), 136 items
+    (40, 8500, 16, 8), (200, 8300, 64, 8), (700, 8200, 32, 8),  # more than 64 key tiles: page ids reloaded
+])
+def test_prefill_workgroups_per_tile(oracle, rows, cached, hq, hk, exact_p):
+    """One request either side of each choice of workgroups per tile, with
+    rows that end inside a quarter or half of a tile; unread slots hold NaN.
+    The oracle checks up to 64 rows spread over the request."""
+    c = W.ragged_prefill_case(1, hq, hk, rows, rows, cached, cached, seed=rows + cached, slack_pages=3)
+    kv = c.kv.reshape(c.num_pages, 16, -1)
+    used = np.zeros((c.num_pages, 16), bool)
+    t = np.arange(rows + cached)
+    used[c.pages[t // 16], t % 16] = True
+    kv[~used] = 0x7FC0
+    got = run_prefill(c, exact_p=exact_p)
+    pick = np.unique(np.r_[0, rows - 1, np.linspace(0, rows - 1, 62).astype(int)])
+    sub = W.PagedCase(hq=hq, hk=hk, page=c.page, pos=c.pos[pick], seq=c.seq[pick], ragged=1, indptr=c.indptr,
+                      pages=c.pages, num_pages=c.num_pages, qkv=c.qkv[pick], kv=c.kv)
+    assert_close(got[pick], oracle_paged(oracle, sub), what=f"{rows} rows over {cached}")
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("q_len,kv_len,batch", [
+    (16, 40, 1), (513, 600, 1), (1024, 1000, 1), (1025, 1102, 1), (520, 520, 2),  # 4, 2, 2, 1, 1 workgroups per tile
+    (1100, 1024, 2),  # 288 items: 32 past a round, split by keys with a workspace, as row halves without
+])
+def test_dit_workgroups_per_tile(oracle, q_len, kv_len, batch, causal):
+    """DiT calls either side of each choice, with and without a workspace,
+    against the oracle on up to 64 rows of the last problem."""
+    c = W.dense_case(32, 8, q_len, kv_len, causal, batch=batch, seed=q_len + kv_len)
+    whole, ws = run_dense(c), run_dense_ws(c)
+    assert_close(ws, whole, what="workspace vs none")
+    if causal:
+        n = min(64, q_len)
+        want = oracle.dense_attend(np.ascontiguousarray(c.q[-1, :n]), np.ascontiguousarray(c.k[-1]),
+                                   np.ascontiguousarray(c.v[-1]), n, kv_len, c.q_stride, 32, 8, 1, c.scale_log2,
+                                   nthreads=16)
+        assert_close(whole[-1][:n], want, what="first rows, causal")
+        if q_len > kv_len:  # rows past the keys see all of them
+            n = q_len - kv_len
+            want = oracle.dense_attend(np.ascontiguousarray(c.q[-1, -n:]), np.ascontiguousarray(c.k[-1]),
+                                       np.ascontiguousarray(c.v[-1]), n, kv_len, c.q_stride, 32, 8, 0, c.scale_log2,
+                                       nthreads=16)
+            assert_close(whole[-1][-n:], want, what="last rows, causal")
+    else:
+        pick = np.unique(np.r_[0, q_len - 1, np.linspace(0, q_len - 1, 62).astype(int)])
+        want = oracle.dense_attend(np.ascontiguousarray(c.q[-1, pick]), np.ascontiguousarray(c.k[-1]),
+                                   np.ascontiguousarray(c.v[-1]), len(pick), kv_len, c.q_stride, 32, 8, 0,
+                                   c.scale_log2, nthreads=16)
+        assert_close(whole[-1][pick], want, what="picked rows")
+
+
 @pytest.mark.parametrize("hq,hk,page", [(32, 8, 16), (16, 16, 16), (16, 8, 12), (64, 8, 16), (8, 4, 3)])
 def test_prefill_exact_p_parity(oracle, hq, hk, page):
     """The plan's exact_p (P carried as two bf16 terms through P.V) on every
