@@ -51,12 +51,24 @@ int resident_tiled_groups() {
 // on 256 CUs), down to 256. Measured on MI355X over seven bucket shapes: a
 // 128-session MHA tick (4096 row x head pairs) runs best at 1024, buckets of
 // 128-512 pairs best at 256-384 (the 64-row GQA talker: 59.5 us at 256
-// against 64.0 at 512), and 128-key splits were slower in every shape.
+// against 64.0 at 512), and 128-key splits were slower in every one of these.
+//
+// Short launches, where the combine launch and idle CUs weigh most (us per
+// layer, replayed graph, 16q/8kv unless said):
+// - rows of at most 512 keys, one per split, once that gives one workgroup per
+//   CU: no partials and no combine. 512 against 256 keys: 32 rows 12.5 / 14.9,
+//   64 rows 20.3 / 22.3, 96 rows 25.6 / 29.2, 32 MHA rows 27.6 / 36.5.
+// - few workgroups: 128 keys, so that a wave has one tile and the keys spread
+//   over more CUs. 128 against 256 keys: 4 rows of up to 512 keys 7.9 / 9.6, 8 of
+//   2400 15.6 / 17.0, 16 of 1200 15.2 / 17.6; 2 MHA rows of 3000 (1536 workgroups)
+//   21.7 / 20.8, 8 GQA rows of 5000 (2560) 24.8 / 24.4.
 int pick_chunk(int rows, int hk, int max_len) {
+  const long long units = (long long)rows * hk;
+  if (max_len > 256 && max_len <= 512 && units >= 256) return 512;
+  if (max_len > 256 && units * (((long long)max_len + 127) / 128) <= 1280) return 128;
   int chunk = 1024;
   while (chunk > 256) {
-    const long long units = (long long)rows * hk * (((long long)max_len + chunk - 1) / chunk);
-    if (units >= 4096) break;
+    if (units * (((long long)max_len + chunk - 1) / chunk) >= 4096) break;
     chunk /= 2;
   }
   return chunk;

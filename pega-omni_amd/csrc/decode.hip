@@ -946,12 +946,23 @@ __global__ __launch_bounds__(64) void decode_combine(DecodeArgs a) {
   a.out[hh * kHead + d + 64] = (bf16_t)f2bf(num1 / den);
 }
 
-// Heads per workgroup: the most that still leaves about 4 workgroups per CU.
+// Heads per workgroup. Eight (1 KiB runs) for long splits that leave about 8
+// workgroups per CU; else four where they leave one per CU, two for a few
+// rows, one for a handful of short ones: a narrower group reads 128-byte runs
+// and loads its scales once per head, a wider one leaves CUs idle. Fused calls
+// of 32 heads, lengths from a tenth of max_len to max_len, the plan's splits,
+// us per layer at 1 / 2 / 4 / 8 heads:
+//   max_len 3000: 1 row 10.1 / 10.7 / 13.5 / 19.6, 5 rows 30.7 / 26.3 / 23.6 / 22.5,
+//     16 rows 69.1 / 52.1 / 48.6 / 46.7, 48 rows 191 / 138 / 123 / 128, 64 rows
+//     (384-key splits) 216 / 161 / 149 / 151, 128 rows (768-key splits) best at 8;
+//   max_len 400: 4 rows 10.4 / 10.9 / 14.1 / 19.3, 16 rows 20.3 / 15.7 / 15.3 / 20.8.
+// (Before: the widest group that leaves 2048 workgroups, so 1 head up to ten rows.)
 static int fp8_heads_per_group(const DecodeArgs& a, int rows) {
   if (a.group_heads) return a.group_heads;
-  for (int h = 8; h > 1; h >>= 1)
-    if (a.hk % h == 0 && (int64_t)rows * (a.hk / h) * a.splits >= 2048) return h;
-  return 1;
+  const auto groups = [&](int h) { return a.hk % h == 0 ? (int64_t)rows * (a.hk / h) * a.splits : 0; };
+  if (a.chunk >= 512 && groups(8) >= 2048) return 8;
+  if (groups(4) >= 256) return 4;
+  return groups(2) >= 192 ? 2 : 1;
 }
 
 // Dynamic LDS the FP8 launch reserves and leaves unused. With the kernel's

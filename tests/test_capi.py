@@ -41,6 +41,18 @@ def test_decode_plan_shapes():
     assert p2.chunk == 256 and p2.splits == 4
 
 
+@pytest.mark.parametrize("rows,hk,max_len,chunk", [
+    (4, 8, 256, 256), (4, 8, 257, 128), (31, 8, 512, 128), (32, 8, 512, 512), (32, 8, 513, 256), (512, 8, 513, 1024),
+    (16, 8, 1280, 128), (16, 8, 1281, 256), (1, 32, 5120, 128), (1, 32, 5121, 256), (64, 8, 2400, 256),
+])
+def test_decode_plan_short_launches(rows, hk, max_len, chunk):
+    """One split per row for rows of at most 512 keys that give a workgroup per
+    CU (256), 128-key splits up to 1280 workgroups, the long-launch rule beyond."""
+    p = oa.decode_plan(rows, 2 * hk, hk, 16, max_len)
+    assert p.chunk == chunk and p.splits == -(-max_len // chunk)
+    assert p.workspace_bytes == (rows * 2 * hk * p.splits * 129 * 4 if p.splits > 1 else 0)
+
+
 @pytest.mark.parametrize("rows,chunk", [(32, 256), (64, 384), (128, 768), (256, 1024), (1, 256)])
 def test_decode_plan_fp8_picks_the_fp8_split(rows, chunk):
     """The FP8 plan's split size: the largest of 1024/768/512/384 keys giving
