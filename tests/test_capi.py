@@ -42,7 +42,7 @@ def test_decode_plan_shapes():
 
 
 @pytest.mark.parametrize("rows,hk,max_len,chunk", [
-    (4, 8, 256, 256), (4, 8, 257, 128), (31, 8, 512, 128), (32, 8, 512, 512), (32, 8, 513, 256), (512, 8, 513, 1024),
+    (4, 8, 256, 256), (4, 8, 257, 128), (31, 8, 512, 128), (32, 8, 512, 512), (32, 8, 513, 128), (33, 8, 513, 256), (512, 8, 513, 1024),
     (16, 8, 1280, 128), (16, 8, 1281, 256), (1, 32, 5120, 128), (1, 32, 5121, 256), (64, 8, 2400, 256),
 ])
 def test_decode_plan_short_launches(rows, hk, max_len, chunk):
