@@ -275,15 +275,20 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   else
     lim = row_ok ? (a.causal ? min(t.len, t.qpos0 + p + 1) : t.len) : 0;
 
-  // Q^T as the B operand: K-step kk holds dims 16 kk + 8 h .. + 7 of row r.
-  bf16x8 qf[8];
-  {
-    const bf16_t* qp = t.q + (int64_t)(row_ok ? p : 0) * a.q_stride + (int64_t)head * kHead + 8 * h;
+  // Q goes through LDS too: each wave's 32 rows by LDS DMA into its 8 KiB of
+  // the second tile buffer (free until the key loop), four whole rows per load
+  // with K's swizzle, and from there into registers as the B operand. (As
+  // 16-byte loads per lane each instruction touched 32 rows, and the eight
+  // waves' Q loads held up the first tile's by 0.5-1 us.) Rows past the tile
+  // read row 0, then become zero.
+  bf16_t* q_lds = smem1 + wave_u * 32 * kHead;
+  if (active) {
 #pragma unroll
-    for (int kk = 0; kk < 8; ++kk) {
-      uint4 u = ldg16(qp + 16 * kk);  // rows past the tile read row 0, then become zero
-      if (!row_ok) u = make_uint4(0, 0, 0, 0);
-      qf[kk] = as_bf16x8(u);
+    for (int i = 0; i < 8; ++i) {
+      const int rq = rb * 32 + 4 * i + (lane >> 4), pq = rq / G;
+      dma_global16(t.q + (int64_t)(pq < t.nq ? pq : 0) * a.q_stride + (int64_t)(kvh * G + rq % G) * kHead +
+                       8 * ((lane & 15) ^ (rq & 15)),
+                   q_lds + 4 * i * kHead);
     }
   }
 
@@ -414,6 +419,15 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   if (SRC == kPagedWave && s_hi > s_lo) pids = wave_pages(s_lo);
   if (s_hi > s_lo) issue_tile(s_lo, smem0);
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), other counters free
+  asm volatile("" ::: "memory");       // the reads of Q stay after the wait
+  // Q^T: K-step kk holds dims 16 kk + 8 h .. + 7 of row r.
+  bf16x8 qf[8];
+#pragma unroll
+  for (int kk = 0; kk < 8; ++kk) {
+    uint4 u = *reinterpret_cast<const uint4*>(q_lds + (k_lane ^ (16 * kk)));
+    if (!row_ok) u = make_uint4(0, 0, 0, 0);
+    qf[kk] = as_bf16x8(u);
+  }
   __syncthreads();
   // One key tile: load the next tile into `nxt`, compute this wave's MB 32-key
   // blocks of it (all four, or its share) from `cur`. The next tile's DMAs go
