@@ -59,13 +59,17 @@ int resident_tiled_groups() {
 //   CU: no partials and no combine. 512 against 256 keys: 32 rows 12.5 / 14.9,
 //   64 rows 20.3 / 22.3, 96 rows 25.6 / 29.2, 32 MHA rows 27.6 / 36.5.
 // - few workgroups: 128 keys, so that a wave has one tile and the keys spread
-//   over more CUs. 128 against 256 keys: 4 rows of up to 512 keys 7.9 / 9.6, 8 of
-//   2400 15.6 / 17.0, 16 of 1200 15.2 / 17.6; 2 MHA rows of 3000 (1536 workgroups)
-//   21.7 / 20.8, 8 GQA rows of 5000 (2560) 24.8 / 24.4.
-int pick_chunk(int rows, int hk, int max_len) {
+//   over more CUs, while all of them still run at once: up to 512, or 256 for
+//   MHA, whose kernel holds two register tiles, and for rows of more than eight
+//   such splits, whose merge grows. 128 against 256 keys: 4 rows of up
+//   to 512 keys 7.9 / 9.6, 1 row of 2400 7.7 / 9.8, 8 of 1000 10.2 / 10.6, 2 MHA
+//   rows of 400 (hk = 32) 8.8 / 9.7; past it, fused with the rotary, 8 rows of 32q/8kv
+//   518-2468 (1280 workgroups) 26.4 / 21.6, 3 MHA rows of 1139-1544 (hk = 16, 624)
+//   19.1 / 17.1, 3 rows of 1364-1621 (312, 13 splits) 11.5 / 10.9.
+int pick_chunk(int rows, int hq, int hk, int max_len) {
   const long long units = (long long)rows * hk;
   if (max_len > 256 && max_len <= 512 && units >= 256) return 512;
-  if (max_len > 256 && units * (((long long)max_len + 127) / 128) <= 1280) return 128;
+  if (max_len > 256 && units * (((long long)max_len + 127) / 128) <= (hq == hk || max_len > 1024 ? 256 : 512)) return 128;
   int chunk = 1024;
   while (chunk > 256) {
     if (units * (((long long)max_len + chunk - 1) / chunk) >= 4096) break;
@@ -190,7 +194,7 @@ static int decode_plan_fill(int rows, int hq, int hk, int page, int max_len, int
   if (G != 1 && G != 2 && G != 4) return fail(OMNI_ATTN_EUNSUPPORTED, "decode_plan: hq/hk=%d not in {1,2,4}", G);
   if (page <= 0) return fail(OMNI_ATTN_EINVAL, "decode_plan: page=%d", page);
   if (max_len <= 0) return fail(OMNI_ATTN_EINVAL, "decode_plan: max_len=%d", max_len);
-  int chunk = chunk_hint > 0 ? chunk_hint : fp8 ? pick_chunk_fp8(rows, hk, max_len) : pick_chunk(rows, hk, max_len);
+  int chunk = chunk_hint > 0 ? chunk_hint : fp8 ? pick_chunk_fp8(rows, hk, max_len) : pick_chunk(rows, hq, hk, max_len);
   if (chunk % 128 != 0) return fail(OMNI_ATTN_EINVAL, "decode_plan: chunk=%d is not a multiple of 128", chunk);
   plan->rows = rows;
   plan->hq = hq;

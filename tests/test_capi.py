@@ -41,16 +41,19 @@ def test_decode_plan_shapes():
     assert p2.chunk == 256 and p2.splits == 4
 
 
-@pytest.mark.parametrize("rows,hk,max_len,chunk", [
-    (4, 8, 256, 256), (4, 8, 257, 128), (31, 8, 512, 128), (32, 8, 512, 512), (32, 8, 513, 128), (33, 8, 513, 256), (512, 8, 513, 1024),
-    (16, 8, 1280, 128), (16, 8, 1281, 256), (1, 32, 5120, 128), (1, 32, 5121, 256), (64, 8, 2400, 256),
+@pytest.mark.parametrize("rows,hq,hk,max_len,chunk", [
+    (4, 16, 8, 256, 256), (4, 16, 8, 257, 128), (16, 16, 8, 512, 128), (17, 16, 8, 512, 256), (32, 16, 8, 512, 512),
+    (32, 16, 8, 513, 256), (512, 16, 8, 513, 1024), (8, 32, 8, 1024, 128), (4, 32, 8, 1025, 256),
+    (3, 16, 8, 1280, 128), (3, 16, 8, 1281, 256), (1, 16, 8, 4096, 128), (1, 16, 8, 4097, 256),
+    (2, 32, 32, 512, 128), (2, 32, 32, 513, 256), (7, 32, 32, 512, 256), (8, 32, 32, 512, 512), (64, 16, 8, 2400, 256),
 ])
-def test_decode_plan_short_launches(rows, hk, max_len, chunk):
+def test_decode_plan_short_launches(rows, hq, hk, max_len, chunk):
     """One split per row for rows of at most 512 keys that give a workgroup per
-    CU (256), 128-key splits up to 1280 workgroups, the long-launch rule beyond."""
-    p = oa.decode_plan(rows, 2 * hk, hk, 16, max_len)
+    CU (256), 128-key splits up to 512 workgroups (256 for MHA and beyond
+    eight splits), the long-launch rule past that."""
+    p = oa.decode_plan(rows, hq, hk, 16, max_len)
     assert p.chunk == chunk and p.splits == -(-max_len // chunk)
-    assert p.workspace_bytes == (rows * 2 * hk * p.splits * 129 * 4 if p.splits > 1 else 0)
+    assert p.workspace_bytes == (rows * hq * p.splits * 129 * 4 if p.splits > 1 else 0)
 
 
 @pytest.mark.parametrize("rows,chunk", [(32, 256), (64, 384), (128, 768), (256, 1024), (1, 256)])
