@@ -214,9 +214,12 @@ __global__ __launch_bounds__(64 * kMimiWaves) void mimi_attend64(ShortArgs a) {
 #pragma unroll
       for (int i = 1; i < NI; ++i) mx = fmaxf(mx, sc[i]);
       mx = across_rows8<true>(mx);
-      const float mn = fmaxf(m[j], mx);
-      const float corr = fast_exp2(m[j] - mn);
-      m[j] = mn;
+      const float mo = m[j];
+      m[j] = fmaxf(mo, mx);
+      // Slots whose scores are all -inf (infinite keys) weigh 0: -inf less -inf
+      // would make this wave's share NaN beside another wave's finite one.
+      const float mn = m[j] == -INFINITY ? 0.f : m[j];
+      const float corr = fast_exp2(mo - mn);
       float ps = 0.f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) acc[j][e] *= corr;

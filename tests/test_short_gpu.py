@@ -74,6 +74,28 @@ def test_mimi_attend_rows_of_a_session(oracle, T, context):
     assert_close(got[:rows][keep], want[:rows][keep], what="mimi_attend")
 
 
+@pytest.mark.parametrize("first,count", [(16, 16), (112, 16), (144, 16)])
+def test_mimi_attend_slots_of_infinite_keys(oracle, first, count):
+    """All slots of a wave's trip score -inf (the second wave, the last wave, a wave's
+    second trip): they weigh 0 and the result is that of the other slots."""
+    c = mimi_case(10, sessions=2, T=2, heads=3, context=250)
+    c["pos"] = np.array([100, 124], np.int32)  # not past the ring: slot t is key t
+    slot = 2 * 3 * 64
+    c["qkv"].view(np.uint16)[:] = c["qkv"].view(np.uint16) & 0x7FFF  # q above zero: -inf keys score -inf
+    state = c["state"].view(np.uint16)
+    for line in c["lines"]:
+        at = int(line) * c["stride"] // 2
+        for t in range(first, first + count):
+            state[at + t * slot:at + t * slot + slot // 2] = 0xFF80
+    args = (c["lines"], c["state"], c["rows"], 2, 3, 0.125, 250, c["stride"])
+    want = oracle.mimi_attend(c["qkv"], c["pos"], *args)
+    out = torch.zeros(c["rows"], 3 * 64, dtype=torch.bfloat16, device="cuda")
+    oa.mimi_attend(dev_bits(c["qkv"]), dev_i32(c["pos"]), dev_i32(c["lines"]), torch.from_numpy(c["state"]).cuda(), out,
+                   c["rows"], 2, 3, 0.125, 250, c["stride"])
+    torch.cuda.synchronize()
+    assert_close(host_bits(out), want, what="mimi_attend")
+
+
 @pytest.mark.parametrize("seed,sessions,heads,pos_hi", [(4, 4, 4, 200), (5, 64, 16, 1000), (6, 3, 2, 3)])
 def test_codec_attention(oracle, seed, sessions, heads, pos_hi):
     c = codec_case(seed, sessions=sessions, heads=heads, pos_hi=pos_hi)
