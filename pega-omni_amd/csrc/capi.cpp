@@ -424,7 +424,9 @@ int omni_attn_prefill_run(const omni_attn_prefill_plan* plan, const void* qkv, c
   a.hk = plan->hk;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.exact_p = plan->exact_p;
-  a.subs = omni::tiled_subs(items, resident_tiled_groups());
+  const int resident = resident_tiled_groups();
+  a.quarters = omni::tiled_quarters(items, resident);
+  a.halved = omni::prefill_halves(items, resident);
   const int rc = omni::launch_prefill(a, (int)items, as_stream(stream));
   if (rc == -2) return fail(OMNI_ATTN_EUNSUPPORTED, "prefill_run: shape not implemented");
   if (rc != 0) return fail(OMNI_ATTN_ELAUNCH, "prefill_run: launch failed: %s", hipGetErrorString(omni::g_launch_status));
@@ -493,10 +495,9 @@ int dit_prepare(const void* q, const void* k, const void* v, void* out, int q_le
 }
 
 int dit_launch(omni::TiledArgs& a, int batch, void* stream) {
-  a.subs = 1;
-  if (a.split_k == 0 && a.halved == 0) {
+  if (a.split_k == 0) {
     const int per_tile = omni::kTiledRows / (a.hq / a.hk);
-    a.subs = omni::tiled_subs((long long)((a.q_len + per_tile - 1) / per_tile) * a.hk * batch, resident_tiled_groups());
+    a.quarters = omni::tiled_quarters((long long)((a.q_len + per_tile - 1) / per_tile) * a.hk * batch, resident_tiled_groups());
   }
   const int rc = omni::launch_dit(a, batch, as_stream(stream));
   if (rc == -2) return fail(OMNI_ATTN_EUNSUPPORTED, "hidream_attend: shape not implemented");
@@ -540,7 +541,9 @@ int omni_hidream_attend_ws(const void* q, const void* k, const void* v, void* ou
   if ((reinterpret_cast<uintptr_t>(workspace) & 15) != 0)
     return fail(OMNI_ATTN_EINVAL, "hidream_attend: workspace must be 16-byte aligned");
   int items = 0;
-  omni::dit_split(a, batch, resident_tiled_groups(), &items, &a.split_from, &a.split_k);
+  const int resident = resident_tiled_groups();
+  omni::dit_split(a, batch, resident, &items, &a.split_from, &a.split_k);
+  if (items < resident) a.halved = omni::dit_halves(a, batch, resident);  // no split below a round
   const int64_t need = (int64_t)(items - a.split_from) * a.split_k * omni::kSegmentBytes;
   if (need > workspace_bytes)
     return fail(OMNI_ATTN_EWORKSPACE, "hidream_attend: the split needs %lld workspace bytes, got %lld",

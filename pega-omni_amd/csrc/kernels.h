@@ -97,13 +97,13 @@ struct TiledArgs {
   // chunk: O[128 rows][128] then (m, l)[128 rows]); 0 chunks = no split.
   int split_from, split_k;
   float* ws;
-  // Row halves (dense, no split): the last `halved` items run as two
-  // workgroups of kTiledRows / 2 packed rows each; 0 = none.
+  // Row halves (no split): the last `halved` items (prefill: all or none) run
+  // as two workgroups of kTiledRows / 2 packed rows each; 0 = none.
   int halved;
+  // All items run as four workgroups of a quarter of the rows each (no split).
+  int quarters;
   // Prefill with P carried as two bf16 terms (hi + lo) through P.V.
   int exact_p;
-  // Workgroups per tile (1, 2 or 4; 2 and 4 only without split and halves).
-  int subs;
 };
 
 // Packed (position, head) query rows per MFMA tile: one 8-wave workgroup, one per CU.
@@ -158,8 +158,10 @@ int launch_rope(const RopeArgs& a, int mode, hipStream_t stream);
 int launch_dit(const TiledArgs& a, int batch, hipStream_t stream);
 // Items and the tail split launch_dit would use for a call (split_k = 0: none).
 void dit_split(const TiledArgs& a, int batch, int resident, int* items, int* split_from, int* split_k);
-// Workgroups per tile (TiledArgs::subs) for a call of `items` tiles.
-int tiled_subs(long long items, int resident);
+// Whether a call of `items` tiles should run them as row quarters, and the
+// items launch_prefill should run as row halves otherwise (all or none).
+bool tiled_quarters(long long items, int resident);
+int prefill_halves(long long items, int resident);
 // Items launch_dit should run as row halves when no split is used (0: none).
 int dit_halves(const TiledArgs& a, int batch, int resident);
 

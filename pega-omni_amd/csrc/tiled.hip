@@ -24,7 +24,6 @@
 //     LDS reads (ds_read_b64_tr_b16) per MFMA.
 // LDS layouts keep the MFMA operand reads conflict-free (see kTileElems).
 #include <algorithm>
-#include <type_traits>
 
 #include "common.h"
 #include "kernels.h"
@@ -133,36 +132,48 @@ struct Tile {
   int64_t per_slot;          // paged: elements per slot
 };
 
-// SUBS: workgroups per tile. 1: the eight waves own the tile's eight 32-row
-// blocks and each sees every key. 2 or 4: a workgroup takes 128 or 64 of the
-// tile's rows, waves w and w + 8 / SUBS own the same 32 rows, and each takes
-// its share (64 or 32 keys) of every 128-key tile; their partial (m, l, O)
-// merge in LDS at the end. For calls of too few tiles to fill the GPU.
+// Tiles of calls, or of last rounds, of too few tiles to fill the GPU run as
+// several workgroups of fewer rows. A row is computed as in a whole tile, so
+// its bits do not depend on which form its tile takes.
+// kHalves: two workgroups of kBM / 2 packed rows each (prefill: every tile;
+// DiT: the last `halved`). Waves 0..3 (one per SIMD) compute the first half,
+// waves 4..7 the second, and all eight load the K/V tiles.
+// kQuarters: four workgroups of kBM / 4 rows, two 32-row blocks of four waves
+// each: wave kg of a block takes keys 32 kg .. + 31 of a tile in S and dims
+// 32 kg .. + 31 in P.V (quarter_step).
+constexpr int kWhole = 0, kHalves = 1, kQuarters = 2;
 static_assert(kDmas == 8, "one DMA per K-step of the S stage");
 
 // Key sources: dense K and V; paged with pages that are multiples of the 16
 // rows a wave loads (a wave's rows of a tile lie in one page); any other page.
 constexpr int kDense = 0, kPagedWave = 1, kPagedLane = 2;
 
-template <int G, int SRC, int SUBS = 1, bool HALVES = false, bool EXACT = false>
+template <int G, int SRC, int FORM = kWhole, bool EXACT = false>
 __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items, int ntiles) {
   constexpr bool PAGED = SRC != kDense;
+  constexpr int PARTS = FORM == kQuarters ? 4 : FORM == kHalves ? 2 : 1;
   // DiT, XCD-aware order: workgroup id i runs on XCD i % 8; give each XCD a
   // contiguous block of work items so the tiles sharing one K/V head (and
   // batch) share that XCD's L2.
   // Prefill: the work list gives each XCD a range of (tile, kv head) items,
   // ordered so the workgroups resident on an XCD share one (sequence, kv
   // head) and its K/V stays in that XCD's L2; workgroup i takes item
-  // start[i % 8] + i / 8 (/ SUBS) of its XCD's range.
+  // start[i % 8] + i / 8 (/ PARTS) of its XCD's range.
   // DiT tail split: the first split_from items run whole, then every later
   // item runs as split_k key chunks (workgroups dispatched after all whole
   // items, so they fill the last round), each with its own XCD-aware order.
-  // DiT row halves (HALVES): the last `halved` items run as two workgroups
-  // of kBM / 2 packed rows (as SUBS = 2), in the same order as the split
+  // DiT row halves: the last `halved` items, in the same order as the split
   // chunks.
-  int idx, chunk = -1, sub = 0;
-  int subs = SUBS;  // workgroups this tile runs as
-  if constexpr (HALVES) {
+  int idx, chunk = -1, part = -1;
+  if constexpr (PAGED) {
+    // XCD x's range starts at header entry x, which the plan makes
+    // x (items / 8) + min(x, items % 8): computed, not read, so the item is
+    // the first load of the chain item -> sequence -> page ids -> K.
+    const int x = blockIdx.x & 7, k = blockIdx.x >> 3, nth = k / PARTS;
+    if (nth >= (items >> 3) + (x < (items & 7))) return;
+    idx = x * (items >> 3) + min(x, items & 7) + nth;
+    if constexpr (PARTS > 1) part = PARTS - 1 - k % PARTS;  // a tile's later rows see more keys
+  } else if constexpr (FORM == kHalves) {
     const int halves_from = items - a.halved;
     const int whole8 = ((halves_from + 7) >> 3) << 3;
     if ((int)blockIdx.x < whole8) {
@@ -176,10 +187,9 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       const int u = (b2 & 7) * per + (b2 >> 3);
       if (u >= units) return;
       idx = halves_from + (u >> 1);
-      sub = u & 1;
-      subs = 2;
+      part = u & 1;
     }
-  } else if (!PAGED && a.split_k > 0) {
+  } else if (FORM == kWhole && a.split_k > 0) {
     const int whole8 = ((a.split_from + 7) >> 3) << 3;
     if ((int)blockIdx.x < whole8) {
       const int per = whole8 >> 3;
@@ -194,37 +204,35 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       idx = a.split_from + u / a.split_k;
       chunk = u % a.split_k;
     }
-  } else if (PAGED) {
-    // XCD x's range starts at header entry x, which the plan makes
-    // x (items / 8) + min(x, items % 8): computed, not read, so the item is
-    // the first load of the chain item -> sequence -> page ids -> K.
-    const int x = blockIdx.x & 7, k = blockIdx.x >> 3, j = k / SUBS;
-    if (j >= (items >> 3) + (x < (items & 7))) return;
-    idx = x * (items >> 3) + min(x, items & 7) + j;
-    sub = SUBS - 1 - k % SUBS;  // a tile's later rows see more keys
   } else {
-    const int per = (items * SUBS + 7) >> 3;
-    const int u = (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3));
-    if (u >= items * SUBS) return;
-    idx = u / SUBS;
-    sub = SUBS - 1 - u % SUBS;
+    const int per = (items * PARTS + 7) >> 3;
+    idx = (int)((blockIdx.x & 7) * per + (blockIdx.x >> 3));
+    if (idx >= items * PARTS) return;
+    if constexpr (PARTS > 1) {
+      part = PARTS - 1 - idx % PARTS;
+      idx /= PARTS;
+    }
   }
   const int32_t* item = PAGED ? a.work + kPrefillWorkHeader + 4 * idx : nullptr;
   const int tile = PAGED ? 0 : idx % ntiles;
   const int kvh = PAGED ? item[3] : (idx / ntiles) % a.hk;
   const int b = PAGED ? 0 : idx / (ntiles * a.hk);
   constexpr int kPos = kBM / G;  // positions per tile
-  const int sub_pos = kPos / subs;  // positions of this workgroup: sub_pos * sub ..
+  constexpr int kPartPos = kPos / PARTS;  // and per part
+  // This workgroup's rows end at position `ends` of the tile; a part past a
+  // short tile's end has none.
+  const auto no_rows = [&](int nq) { return part > 0 && kPartPos * part >= nq; };
+  const auto ends = [&](int nq) { return part < 0 ? nq : min(nq, kPartPos * (part + 1)); };
 
   Tile t;
   if constexpr (PAGED) {
     const int s = item[0], first = item[1];
     t.nq = item[2];
+    if (no_rows(t.nq)) return;
     t.pos = a.pos + first;
     t.q = a.q + (int64_t)first * a.q_stride;
     t.out = a.out + (int64_t)first * a.hq * kHead;
-    if (sub_pos * sub >= t.nq) return;  // a short tile: no rows here
-    t.last = t.pos[min(t.nq, sub_pos * (sub + 1)) - 1] + 1;
+    t.last = t.pos[ends(t.nq) - 1] + 1;
     t.len = t.last;
     t.pg = a.pages + a.indptr[s];
     t.per_slot = 2LL * a.hk * kHead;
@@ -234,11 +242,11 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   } else {
     const int q0 = tile * kPos;
     t.nq = min(kPos, a.q_len - q0);
+    if (no_rows(t.nq)) return;
     t.q = a.q + b * a.q_bstride + (int64_t)q0 * a.q_stride;
     t.out = a.out + b * a.out_bstride + (int64_t)q0 * a.hq * kHead;
     t.len = *a.kv_len_at;
-    if (sub_pos * sub >= t.nq) return;  // a short tile: no rows here
-    t.last = a.causal ? min(t.len, q0 + min(t.nq, sub_pos * (sub + 1))) : t.len;
+    t.last = a.causal ? min(t.len, q0 + ends(t.nq)) : t.len;
     t.qpos0 = q0;
     t.kv_stride = (int64_t)a.hk * kHead;
     t.kbase = a.k + b * a.kv_bstride + (int64_t)kvh * kHead;
@@ -258,16 +266,17 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = lane & 31, h = lane >> 5;
 
-  // This lane's query column: packed row r of the tile, in 32-row block rb.
-  // The wave's share of a key tile: its kg-th part of `subs`.
+  // This lane's query column: packed row r of the tile, in 32-row block rb
+  // (kQuarters: shared by four waves, one per SIMD, kg = 0..3).
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-  const int blocks = kWaves / subs;  // 32-row blocks of this workgroup
-  const int rb = blocks * sub + wave_u % blocks, kg = wave_u / blocks;
+  const int rb = FORM == kQuarters ? 2 * part + (wave_u >> 2) : wave_u;
+  const int kg = wave_u & 3;
   const int r = rb * 32 + j;
-  const int p = r / G, head = kvh * G + r % G;
-  // Waves none of whose 32 rows is a position of the tile (a short last
-  // tile) only load K/V tiles and meet the barriers (wave-uniform).
-  const bool active = (32 * rb) / G < t.nq;
+  const int p = r / G;
+  // Waves outside this workgroup's half, and waves none of whose 32 rows is a
+  // position of the tile (a short last tile), only load K/V tiles and meet
+  // the barriers (wave-uniform).
+  const bool active = (FORM != kHalves || part < 0 || (wave_u >> 2) == part) && (32 * rb) / G < t.nq;
   const bool row_ok = p < t.nq && active;
   int lim;  // keys this row sees
   if constexpr (PAGED)
@@ -399,7 +408,6 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     for (int e = 0; e < 16; ++e) o[md][e] = 0.f;
   float m = -INFINITY, l = 0.f;
   const float sl2 = a.scale_log2;
-  const float grow_by = subs == 1 ? 8.f : 0.f;
 
   // Per-lane LDS bases (elements). S's A operand: K row 32 mb + j, chunk
   // 2 kk + h, in slot (2 kk + h) ^ (j & 15): elem = (k_lane ^ 16 kk) + 4096 mb.
@@ -429,34 +437,31 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     qf[kk] = as_bf16x8(u);
   }
   __syncthreads();
-  // One key tile: load the next tile into `nxt`, compute this wave's MB 32-key
-  // blocks of it (all four, or its share) from `cur`. The next tile's DMAs go
+  // One key tile: load the next tile into `nxt`, compute from `cur`. The next tile's DMAs go
   // out one per K-step of the S stage: issued together at the top of the step,
   // the eight waves' 64 KiB kept the address unit busy and every wave waiting
   // to issue for 0.45-0.75 us of a 3.1 us step, with the matrix cores idle.
-  auto tile_step = [&](auto mb_count, int st, const bf16_t* cur, bf16_t* nxt) __attribute__((always_inline)) {
-    constexpr int MB = decltype(mb_count)::value;
+  auto tile_step = [&](int st, const bf16_t* cur, bf16_t* nxt) __attribute__((always_inline)) {
     if constexpr (SRC != kPagedLane)
       aim_tile(st + 1);
     else if (st + 1 < s_hi)
       issue_tile(st + 1, nxt);
-    const int own = MB == kMB ? 0 : 32 * MB * kg;  // the wave's first key of the tile
-    const int n0 = st * kBN + own;
-    const bf16_t* kt = cur + own * kHead;
-    const bf16_t* vt = cur + kTileElems + own * kHead;  // V tile
+    const int n0 = st * kBN;
+    const bf16_t* kt = cur;
+    const bf16_t* vt = cur + kTileElems;  // V tile
 
-    // S^T = K . Q^T for keys n0 .. n0 + 32 MB - 1: MB interleaved MFMA chains
+    // S^T = K . Q^T for keys n0 .. n0 + kBN - 1: kMB interleaved MFMA chains
     // (32-key blocks mb) over the 8 K-steps, with the K fragments read
     // from LDS two K-steps ahead of use; the stages are pinned in this order.
-    f32x16 sc[MB];
+    f32x16 sc[kMB];
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) sc[mb][e] = 0.f;
-    uint4 kf[8][MB];
+    uint4 kf[8][kMB];
     auto read_k = [&](int kk) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb) kf[kk][mb] = *reinterpret_cast<const uint4*>(kt + (k_lane ^ (16 * kk)) + mb * 4096);
+      for (int mb = 0; mb < kMB; ++mb) kf[kk][mb] = *reinterpret_cast<const uint4*>(kt + (k_lane ^ (16 * kk)) + mb * 4096);
     };
     read_k(0);
     read_k(1);
@@ -464,7 +469,7 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
 #pragma unroll
     for (int kk = 0; kk < 8; ++kk) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
+      for (int mb = 0; mb < kMB; ++mb)
         sc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[kk][mb]), qf[kk], sc[mb], 0, 0, 0);
       if constexpr (SRC != kPagedLane) dma_tile(kk, nxt);
       if (kk + 2 < 8) read_k(kk + 2);
@@ -472,16 +477,16 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     }
 
     // Register e of block mb is key n0 + 32 mb + 8 (e / 4) + 4 h + e % 4.
-    if (__any(n0 + 32 * MB > lim)) {
+    if (__any(n0 + kBN > lim)) {
 #pragma unroll
-      for (int mb = 0; mb < MB; ++mb)
+      for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll
         for (int e = 0; e < 16; ++e)
           if (n0 + 32 * mb + 8 * (e >> 2) + 4 * h + (e & 3) >= lim) sc[mb][e] = -INFINITY;
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+    for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll
       for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[mb][e]);
     {  // lanes l and l ^ 32 hold the two halves of the row's keys
@@ -490,12 +495,9 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     }
     // The running base m moves only when the max grows by more than 8 (log2):
     // p = 2^(s - m) <= 2^8 stays exact in f32 and l, O share the same base,
-    // so the result is unchanged while most tiles skip rescaling O. A wave
-    // that sees only its share of a tile moves its base with every new max:
-    // its first tile holds a row's largest score less often, and p = 1 is the
-    // one value that rounding to bf16 leaves exact.
+    // so the result is unchanged while most tiles skip rescaling O.
     const float mt = mx * sl2;
-    const bool grow = mt > m + grow_by;
+    const bool grow = mt > m + 8.f;
     if (__any(grow)) {
       const float alpha = grow ? fast_exp2(m - mt) : 1.f;
       m = grow ? mt : m;
@@ -512,12 +514,12 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     // three requests of 60-400 rows over 700-3100 keys, four layers; rounded P
     // unchanged. Pinned between the MFMAs by scheduling barriers it is 1-2%
     // slower in both).
-    constexpr int KS = 2 * MB;
-    float ps[4] = {0.f, 0.f, 0.f, 0.f};
+    constexpr int KS = 2 * kMB;
+    float psum = 0.f;  // in key order, whatever the instruction order
     auto exp_one = [&](int ks, int e) __attribute__((always_inline)) {
       const float x = fast_exp2(fmaf(sc[ks >> 1][8 * (ks & 1) + e], sl2, -base));
       sc[ks >> 1][8 * (ks & 1) + e] = x;
-      ps[e & 3] += x;
+      psum += x;
     };
     // EXACT: P = P_hi + P_lo, both bf16 (P_lo = bf16(P - P_hi), P - P_hi exact
     // in f32), and P.V as two MFMAs: P carries 16 significant bits into the
@@ -566,32 +568,186 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       pf = pn;
       if constexpr (EXACT) pfl = pnl;
     }
-    l += (ps[0] + ps[1]) + (ps[2] + ps[3]);
+    l += psum;
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next tile has landed
     __syncthreads();
   };
+  if constexpr (FORM == kQuarters) {
+    // One key tile for the four waves of a row block. S's key blocks and P.V's
+    // dim blocks are independent MFMA chains, so dealing them to four waves
+    // leaves each chain as it is; the row's max is that of the four, exchanged
+    // through LDS; P goes to the other waves through LDS as the operand it is
+    // (the tile's K rows are free once every wave has its scores); and the sum
+    // of the row's p runs on from wave to wave in key order, each wave taking
+    // its turn one barrier after the one before (waves 2 and 3 in the next
+    // step). Three barriers per tile; bound by that chain of exchanges. 257
+    // queries x 4096 keys (32q/8kv, 40 tiles), us: 52.6, as halves 68, as whole
+    // tiles 84. (Slower: V's operands read after the exchange of maxima 54.8, the
+    // turns beside the MFMAs 59, as a pipeline over four steps 53.7. With the
+    // keys shared through P.V and four partial results merged at the end it was
+    // 39, but then a row's bits depend on the form.)
+    __shared__ float s_max[2][4][32], s_sum[2][3][64], s_inv[2][64];
+    const int blk = wave_u >> 2;
+    constexpr int kSteps = 2 * kMB;  // 16-key K-steps of P.V
+    f32x16 pr, ov;                   // the wave's p of the last tile; its dims of O
+#pragma unroll
+    for (int e = 0; e < 16; ++e) ov[e] = pr[e] = 0.f;
+    auto chain = [&](float sum) __attribute__((always_inline)) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sum += pr[e];
+      return sum;
+    };
+    auto quarter_step = [&](int st, bf16_t* cur, bf16_t* nxt) __attribute__((always_inline)) {
+      aim_tile(st + 1);
+      if (!active) {
+#pragma unroll
+        for (int d = 0; d < kDmas; ++d) dma_tile(d, nxt);
+        __syncthreads();
+        __syncthreads();
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        __syncthreads();
+        return;
+      }
+      const bool later = st > s_lo;
+      if (later && kg == 2) s_sum[blk][2][lane] = chain(s_sum[blk][1][lane]);
+      const int n0 = st * kBN + 32 * kg;
+      const bf16_t* kt = cur + 32 * kg * kHead;
+      const bf16_t* vt = cur + kTileElems;
+      f32x16 sc;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) sc[e] = 0.f;
+      uint4 kf[8];
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) kf[kk] = *reinterpret_cast<const uint4*>(kt + (k_lane ^ (16 * kk)));
+      // V's operands too, a K-step beside each MFMA of S (after the exchange of
+      // maxima they would stand before it in the LDS queue).
+      bf16x8 vf[kSteps];
+      auto read_v = [&](int ks) __attribute__((always_inline)) {
+        const bf16_t* vb = vt + (v_lane ^ (32 * kg)) + 16 * ks * kHead;
+        const bf16x4 lo = lds_read_tr(vb);
+        const bf16x4 hi = lds_read_tr(vb + 8 * kHead);
+        vf[ks] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      };
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int kk = 0; kk < 8; ++kk) {
+        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(kf[kk]), qf[kk], sc, 0, 0, 0);
+        dma_tile(kk, nxt);
+        read_v(kk);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // Register e is key n0 + 8 (e / 4) + 4 h + e % 4.
+      if (__any(n0 + 32 > lim)) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (n0 + 8 * (e >> 2) + 4 * h + (e & 3) >= lim) sc[e] = -INFINITY;
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[e]);
+      {
+        const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+        mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+      }
+      if (h == 0) s_max[blk][kg][j] = mx;
+      __syncthreads();  // every score is taken: the maxima are there and K is free
+      if (later && kg == 3) l += chain(s_sum[blk][2][lane]);  // before this tile's base moves
+      mx = fmaxf(fmaxf(s_max[blk][0][j], s_max[blk][1][j]), fmaxf(s_max[blk][2][j], s_max[blk][3][j]));
+      const float mt = mx * sl2;
+      const bool grow = mt > m + 8.f;
+      if (__any(grow)) {
+        const float alpha = grow ? fast_exp2(m - mt) : 1.f;
+        m = grow ? mt : m;
+        l *= alpha;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) ov[e] *= alpha;
+      }
+      const float base = m == -INFINITY ? 0.f : m;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) pr[e] = fast_exp2(fmaf(sc[e], sl2, -base));
+      uint4* pb = reinterpret_cast<uint4*>(cur) + blk * (64 * kSteps);  // [K-step][lane], then P_lo likewise
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        float pv[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pv[e] = pr[8 * i + e];
+        const uint4 hi = __builtin_bit_cast(uint4, pack8(pv));
+        pb[64 * (2 * kg + i) + lane] = hi;
+        if constexpr (EXACT) {
+          float pl[8];
+          widen8(hi, pl);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) pl[e] = pv[e] - pl[e];
+          pb[2 * 64 * kSteps + 64 * (2 * kg + i) + lane] = __builtin_bit_cast(uint4, pack8(pl));
+        }
+      }
+      if (kg == 0) s_sum[blk][0][lane] = chain(0.f);
+      __syncthreads();  // P is there
+      if (kg == 1) s_sum[blk][1][lane] = chain(s_sum[blk][0][lane]);
+      uint4 pf[kSteps], pfl[EXACT ? kSteps : 1];
+#pragma unroll
+      for (int ks = 0; ks < kSteps; ++ks) {
+        pf[ks] = pb[64 * ks + lane];
+        if constexpr (EXACT) pfl[ks] = pb[2 * 64 * kSteps + 64 * ks + lane];
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < kSteps; ++ks) {
+        ov = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks], as_bf16x8(pf[ks]), ov, 0, 0, 0);
+        if constexpr (EXACT) ov = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks], as_bf16x8(pfl[ks]), ov, 0, 0, 0);
+      }
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next tile has landed
+      __syncthreads();
+    };
+    for (int st = s_lo; st < s_hi; st += 2) {
+      quarter_step(st, smem0, smem1);
+      if (st + 1 < s_hi) quarter_step(st + 1, smem1, smem0);
+    }
+    // The last tile's turns of waves 2 and 3, then the row's 1 / l to all four.
+    const bool any = s_hi > s_lo;
+    if (any && active && kg == 2) s_sum[blk][2][lane] = chain(s_sum[blk][1][lane]);
+    __syncthreads();
+    if (active && kg == 3) {
+      if (any) l += chain(s_sum[blk][2][lane]);
+      l += xor_lane(l, 32);
+      s_inv[blk][lane] = 1.f / l;
+    }
+    __syncthreads();
+    bf16_t* rows = smem0 + blk * 32 * kHead;
+    if (active) {
+      const float inv = s_inv[blk][lane];
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        uint2 w;
+        w.x = pack_bf16x2(ov[4 * q4 + 0] * inv, ov[4 * q4 + 1] * inv);
+        w.y = pack_bf16x2(ov[4 * q4 + 2] * inv, ov[4 * q4 + 3] * inv);
+        *reinterpret_cast<uint2*>(rows + j * kHead + 8 * ((4 * kg + q4) ^ (j & 15)) + 4 * h) = w;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // rows 8 kg .. + 7 of the block, whole
+      const int jr = 8 * kg + 4 * i + (lane >> 4), c = lane & 15;
+      const int rr = rb * 32 + jr, pw = rr / G;
+      const uint4 w = *reinterpret_cast<const uint4*>(rows + jr * kHead + 8 * (c ^ (jr & 15)));
+      if (pw < t.nq)
+        *reinterpret_cast<uint4*>(t.out + ((int64_t)pw * a.hq + kvh * G + rr % G) * kHead + 8 * c) = w;
+    }
+    return;
+  }
+
   if (!active) {  // computes nothing: the same loads (its rows of every K/V tile) and barriers
     for (int st = s_lo; st < s_hi; ++st) {
       if (st + 1 < s_hi) issue_tile(st + 1, (st - s_lo) & 1 ? smem0 : smem1);
       __builtin_amdgcn_s_waitcnt(0x0F70);
       __syncthreads();
     }
-    if (SUBS > 1 || (HALVES && subs > 1)) {  // the merge's two
-      __syncthreads();
-      __syncthreads();
-    }
     return;
   }
-  auto key_loop = [&](auto mb_count) __attribute__((always_inline)) {
-    for (int st = s_lo; st < s_hi; st += 2) {  // unrolled by two: buffer addresses are constants
-      tile_step(mb_count, st, smem0, smem1);
-      if (st + 1 < s_hi) tile_step(mb_count, st + 1, smem1, smem0);
-    }
-  };
-  if (HALVES && subs > 1)
-    key_loop(std::integral_constant<int, kMB / 2>{});
-  else
-    key_loop(std::integral_constant<int, kMB / SUBS>{});
+  for (int st = s_lo; st < s_hi; st += 2) {  // unrolled by two: buffer addresses are constants
+    tile_step(st, smem0, smem1);
+    if (st + 1 < s_hi) tile_step(st + 1, smem1, smem0);
+  }
 
   // Register e of block md is dim 32 md + 8 (e / 4) + 4 h + e % 4.
   l += xor_lane(l, 32);
@@ -607,50 +763,6 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
     if (h == 0) *reinterpret_cast<float2*>(seg + kBM * kHead + 2 * r) = make_float2(m, l);
     return;
   }
-  // Waves that share rows exchange their partials through the (now free) tile
-  // buffers: 16 KiB of O per wave, element (md, q4) of lane l at 16-byte slot
-  // 64 (4 md + q4) + l. Wave kg of a row block then merges and stores the
-  // dims of blocks md = kg * 4 / subs .. + 4 / subs - 1.
-  int md_lo = 0, md_n = 4;
-  if constexpr (SUBS > 1 || HALVES) {
-    if (subs > 1) {
-      __shared__ float2 s_ml[kWaves][64];
-      auto region = [&](int w) { return reinterpret_cast<float4*>(w < 4 ? smem0 : smem1) + (w & 3) * 1024; };
-#pragma unroll
-      for (int md = 0; md < 4; ++md)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-          region(wave_u)[64 * (4 * md + q4) + lane] =
-              make_float4(o[md][4 * q4], o[md][4 * q4 + 1], o[md][4 * q4 + 2], o[md][4 * q4 + 3]);
-      s_ml[wave][lane] = make_float2(m, l);
-      __syncthreads();
-      md_n = 4 / subs;
-      md_lo = kg * md_n;
-      float top = -INFINITY;
-      for (int g = 0; g < subs; ++g) top = fmaxf(top, s_ml[wave_u % blocks + g * blocks][lane].x);
-#pragma unroll
-      for (int md = 0; md < 4 / (SUBS > 1 ? SUBS : 2); ++md)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) o[md][e] = 0.f;
-      l = 0.f;
-      for (int g = 0; g < subs; ++g) {
-        const int w = wave_u % blocks + g * blocks;
-        const float2 ml = s_ml[w][lane];
-        const float f = ml.x == -INFINITY ? 0.f : fast_exp2(ml.x - top);
-        l = fmaf(ml.y, f, l);
-#pragma unroll
-        for (int md = 0; md < 4 / (SUBS > 1 ? SUBS : 2); ++md)
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            const float4 v = region(w)[64 * (4 * (md_lo + md) + q4) + lane];
-            o[md][4 * q4 + 0] = fmaf(v.x, f, o[md][4 * q4 + 0]);
-            o[md][4 * q4 + 1] = fmaf(v.y, f, o[md][4 * q4 + 1]);
-            o[md][4 * q4 + 2] = fmaf(v.z, f, o[md][4 * q4 + 2]);
-            o[md][4 * q4 + 3] = fmaf(v.w, f, o[md][4 * q4 + 3]);
-          }
-      }
-    }
-  }
   // Normalise and store. A row that sees no key (*kv_len_at = 0) has l = 0 and
   // O = 0, and stores 0 * (1 / 0) = NaN, as hidream.cu:333-346 does. The rows
   // go through LDS (64 (d / 8) + lane order undone by the read) so that a
@@ -658,31 +770,28 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   // bytes of 32 different rows: 16-byte chunk c of block row j sits in slot
   // c ^ (j & 15) of its row, and the wave alone uses its 8 KiB.
   const float inv = 1.f / l;
-  constexpr int kDims = kHead / SUBS;  // dims this wave stores (half of them in the halves' workgroups)
-  if constexpr (SUBS > 1 || HALVES)
-    if (subs > 1) __syncthreads();  // the merge's reads are over
+  int ln = lane;
+  asm volatile("" : "+v"(ln));  // the addresses below are made here, not held in registers through the key loop
+  const int jn = ln & 31, hn = ln >> 5;
   bf16_t* rows = (wave_u < 4 ? smem0 : smem1) + (wave_u & 3) * 32 * kHead;
 #pragma unroll
-  for (int md = 0; md < 4 / SUBS; ++md)
+  for (int md = 0; md < 4; ++md)
 #pragma unroll
     for (int q4 = 0; q4 < 4; ++q4) {
-      if (HALVES && md >= md_n) break;
-      // dims 32 md + 8 q4 + 4 h .. + 3 of this wave's: half h of chunk 4 md + q4
+      // dims 32 md + 8 q4 + 4 h .. + 3: half h of chunk 4 md + q4
       uint2 w;
       w.x = pack_bf16x2(o[md][4 * q4 + 0] * inv, o[md][4 * q4 + 1] * inv);
       w.y = pack_bf16x2(o[md][4 * q4 + 2] * inv, o[md][4 * q4 + 3] * inv);
-      *reinterpret_cast<uint2*>(rows + j * kHead + 8 * ((4 * md + q4) ^ (j & 15)) + 4 * h) = w;
+      *reinterpret_cast<uint2*>(rows + jn * kHead + 8 * ((4 * md + q4) ^ (jn & 15)) + 4 * hn) = w;
     }
-  // The block's rows, 16-byte chunk by chunk: the wave's own LDS writes, in order.
-  const int chunks = HALVES ? 4 * md_n : kDims / 8;  // 16-byte chunks of a row
+  // The block's rows, four per instruction, a 16-byte chunk per lane.
 #pragma unroll
-  for (int i = 0; i < 8 / SUBS; ++i) {
-    if (HALVES && i >= 2 * md_n) break;
-    const int at = 64 * i + lane, jr = at / chunks, c = at % chunks;
-    const int rr = rb * 32 + jr, pr = rr / G;
+  for (int i = 0; i < 8; ++i) {
+    const int jr = 4 * i + (ln >> 4), c = ln & 15;
+    const int rr = wave_u * 32 + jr, pr = rr / G;
     const uint4 w = *reinterpret_cast<const uint4*>(rows + jr * kHead + 8 * (c ^ (jr & 15)));
     if (pr < t.nq)
-      *reinterpret_cast<uint4*>(t.out + ((int64_t)pr * a.hq + kvh * G + rr % G) * kHead + 32 * md_lo + 8 * c) = w;
+      *reinterpret_cast<uint4*>(t.out + ((int64_t)pr * a.hq + kvh * G + rr % G) * kHead + 8 * c) = w;
   }
 }
 
@@ -753,48 +862,43 @@ __global__ __launch_bounds__(256) void dit_combine(TiledArgs a, int ntiles) {
   *reinterpret_cast<uint4*>(a.out + b * a.out_bstride + ((int64_t)(q0 + p) * a.hq + head) * kHead + d0) = o;
 }
 
-template <int G, int SRC, int SUBS>
-void launch_subs(const TiledArgs& a, int grid, int items, int ntiles, hipStream_t stream) {
-  // Prefill with exact_p set: the hi + lo P.V variant (prefill only; DiT
-  // rounds P to bf16 as hidream.cu does).
-  if (SRC != kDense && a.exact_p)
-    tiled_attn<G, SRC, SUBS, false, SRC != kDense><<<grid, kThreads, 0, stream>>>(a, items, ntiles);
-  else
-    tiled_attn<G, SRC, SUBS><<<grid, kThreads, 0, stream>>>(a, items, ntiles);
-}
-
-template <int G, int SRC>
+// Prefill with exact_p set: the hi + lo P.V variant (prefill only; DiT rounds
+// P to bf16 as hidream.cu does).
+template <int G, int SRC, int FORM>
 void launch_g(const TiledArgs& a, int grid, int items, int ntiles, hipStream_t stream) {
-  if (a.subs == 4)
-    launch_subs<G, SRC, 4>(a, grid, items, ntiles, stream);
-  else if (a.subs == 2)
-    launch_subs<G, SRC, 2>(a, grid, items, ntiles, stream);
+  if (SRC != kDense && a.exact_p)
+    tiled_attn<G, SRC, FORM, SRC != kDense><<<grid, kThreads, 0, stream>>>(a, items, ntiles);
   else
-    launch_subs<G, SRC, 1>(a, grid, items, ntiles, stream);
+    tiled_attn<G, SRC, FORM><<<grid, kThreads, 0, stream>>>(a, items, ntiles);
 }
 
 template <bool PAGED>
-int launch_tiled(const TiledArgs& args, int items, int ntiles, hipStream_t stream) {
+int launch_tiled(const TiledArgs& a, int items, int ntiles, hipStream_t stream) {
   if (items <= 0) return 0;
-  TiledArgs a = args;
-  // Pages that are no multiple of a wave's rows keep one workgroup per tile.
+  // Pages that are no multiple of a wave's rows keep whole tiles.
   const bool lane_pages = PAGED && a.pd.page % kRowsPerWave != 0;
-  if (lane_pages) a.subs = 1;
-  // Prefill: the XCDs' item ranges differ by one, each item `subs` workgroups.
-  int grid = PAGED ? (((items + 7) >> 3) << 3) * a.subs : ((items * a.subs + 7) >> 3) << 3;
-  if (!PAGED && a.split_k > 0)
+  const bool parts = !lane_pages && (PAGED || a.split_k == 0);
+  const int form = parts && a.quarters ? kQuarters : parts && a.halved > 0 ? kHalves : kWhole;
+  int grid = ((items + 7) >> 3) << 3;
+  if (PAGED)
+    grid *= form == kQuarters ? 4 : form == kHalves ? 2 : 1;  // an XCD's items, each as so many workgroups
+  else if (form == kQuarters)
+    grid = ((items * 4 + 7) >> 3) << 3;
+  else if (form == kHalves)
+    grid = (((items - a.halved + 7) >> 3) << 3) + (((a.halved * 2 + 7) >> 3) << 3);
+  else if (a.split_k > 0)
     grid = (((a.split_from + 7) >> 3) << 3) + ((((items - a.split_from) * a.split_k + 7) >> 3) << 3);
-  const bool halves = !PAGED && a.split_k == 0 && a.halved > 0;
-  if (halves) grid = (((items - a.halved + 7) >> 3) << 3) + (((a.halved * 2 + 7) >> 3) << 3);
   switch (a.hq / a.hk) {
 #define OMNI_CASE(G)                                                                       \
   case G:                                                                                  \
-    if (halves)                                                                            \
-      tiled_attn<G, kDense, 1, true><<<grid, kThreads, 0, stream>>>(a, items, ntiles);     \
-    else if (lane_pages)                                                                   \
-      launch_subs<G, PAGED ? kPagedLane : kDense, 1>(a, grid, items, ntiles, stream);      \
+    if (lane_pages)                                                                        \
+      launch_g<G, PAGED ? kPagedLane : kDense, kWhole>(a, grid, items, ntiles, stream);    \
+    else if (form == kQuarters)                                                            \
+      launch_g<G, PAGED ? kPagedWave : kDense, kQuarters>(a, grid, items, ntiles, stream); \
+    else if (form == kHalves)                                                              \
+      launch_g<G, PAGED ? kPagedWave : kDense, kHalves>(a, grid, items, ntiles, stream);   \
     else                                                                                   \
-      launch_g<G, PAGED ? kPagedWave : kDense>(a, grid, items, ntiles, stream);            \
+      launch_g<G, PAGED ? kPagedWave : kDense, kWhole>(a, grid, items, ntiles, stream);    \
     break;
     OMNI_CASE(1)
     OMNI_CASE(2)
@@ -825,26 +929,31 @@ int launch_dit(const TiledArgs& a, int batch, hipStream_t stream) {
   return launch_tiled<false>(a, (int)items, ntiles, stream);
 }
 
-// Workgroups per tile for a call of `items` tiles on `resident` CUs: as many as
-// still fit one round. A workgroup of a half (quarter) of a tile's rows takes
-// 0.68 (0.4-0.5) of a whole one's time, so a second round would lose what the
-// split wins. us per launch, replayed graph, 1 / 2 / 4 workgroups per tile:
-// 187 rows of 16q/8kv (16 tiles) 10.3 / 10.9 / 9.5; three requests of 60-400
-// rows over 700-3100 cached keys, 32q/8kv, exact P (104 tiles) 89 / 61 / 68;
-// 1025 DiT rows over 1102 keys (136 tiles, two rounds when split) 33 / 45 / 50.
-int tiled_subs(long long items, int resident) {
-  if (items * 4 <= resident) return 4;
-  return items * 2 <= resident ? 2 : 1;
-}
+// Calls whose tiles fill at most a quarter of the CUs run each as four
+// workgroups, others of up to half the CUs as two: as many as still fit one
+// round. us per launch, replayed graph, as 1 / 2 / 4 workgroups per tile:
+//   187 rows of 16q/8kv (16 tiles) 9.1 / 9.1 / 8.0; 1000 rows (64) 28.8 / 22.4 /
+//   18.5; 32q/8kv, 600 rows over 500 (80) 29.1 / 21.4 / 26.0; three requests of 60-400
+//   rows over 700-3100 (104) 76 / 53 / 73, exact P 102 / 68 / 88;
+//   short prompts, one or two key tiles: 6 x 187 rows (96) 9.5 / 9.4 / 12.9,
+//   16 x 30 rows (128) 7.0 / 7.0 / 11.1, 14 x 64 rows of 32q/8kv (112) 9.4 / 8.2 / 12.0;
+//   DiT 257 x 334 (40) 13.3 / 10.6 / 9.7; 577 x 660 (80) 21.3 / 17.0 / 26.5.
+// (72 causal tiles of one request of 1100 rows take 31.2 / 23.9 / 20.3: its second
+// round of quarters holds only short walks. 72 equal tiles lose like 80.)
+bool tiled_quarters(long long items, int resident) { return items > 0 && items * 4 <= resident; }
 
-// Without a workspace: when the last round holds at most half the resident
-// workgroups, its items run as row halves (two workgroups each, on twice the
-// CUs); such a round takes about 0.7 of a full round's time.
+int prefill_halves(long long items, int resident) { return items * 2 <= resident ? (int)items : 0; }
+
+// DiT: when the last round holds at most half the resident workgroups, its
+// items run as row halves (two workgroups each, on twice the CUs). A half takes
+// 0.71-0.82 of a whole tile's time (lone rounds of 80-128 tiles). us, whole /
+// halves: 2049 x 2100 (264 tiles) 100.4 / 97.4, 2200 x 2300 (280) 115 / 99.6, the
+// pair of 4352 x 4352 (1088) 560 / 532.
 int dit_halves(const TiledArgs& a, int batch, int resident) {
   const int G = a.hq / a.hk;
   const int ntiles = (a.q_len + kBM / G - 1) / (kBM / G);
   const long long n = (long long)ntiles * a.hk * batch;
-  if (resident <= 0 || n < resident || n > (1LL << 30)) return 0;  // less than a round: tiled_subs
+  if (resident <= 0 || n <= 0 || n > (1LL << 30)) return 0;
   const int rem = (int)(n % resident);
   return 2 * rem > resident ? 0 : rem;
 }
@@ -865,11 +974,8 @@ void dit_split(const TiledArgs& a, int batch, int resident, int* items, int* spl
   *items = (int)n;
   *split_from = (int)n;
   *split_k = 0;
-  // Calls of less than one round split their tiles by rows within the launch
-  // instead (tiled_subs): no partials in memory and no combine launch. 32q/8kv,
-  // us per call, by keys / by rows: 65 queries x 142 keys 17.2 / 11.6, 257 x 334
-  // 22.6 / 13.6, 1000 x 1077 37.8 / 27.5; key splits would win only for few
-  // queries over many keys (257 x 4096 56 / 61), which DiT calls are not.
+  // Calls of less than one round run as row parts within the launch instead
+  // (tiled_quarters, dit_halves): no partials in memory and no combine launch.
   if (resident <= 0 || n < resident || n > (1LL << 30)) return;
   const int rem = (int)(n % resident);
   if (rem == 0 || resident / rem < 2) return;

@@ -385,6 +385,48 @@ def test_dit_workgroups_per_tile(oracle, q_len, kv_len, batch, causal):
         assert_close(whole[-1][pick], want, what="picked rows")
 
 
+@pytest.mark.parametrize("exact_p", [False, True])
+@pytest.mark.parametrize("hq,hk,rows,cached", [(16, 8, 187, 0), (32, 8, 150, 700), (16, 16, 40, 300), (64, 8, 33, 1000)])
+def test_prefill_row_bits_do_not_depend_on_the_call(hq, hk, rows, cached, exact_p):
+    """A request's rows alone (few tiles: row halves), beside others that still
+    leave CUs idle, and in a call of more tiles than CUs (whole tiles): the same
+    bits every time, since each row is computed the same way in all of them."""
+    per = 256 * hk // hq
+    c = W.ragged_prefill_case(2, hq, hk, rows, rows, cached, cached, seed=rows)
+    alone, both = np.flatnonzero(c.seq == 0), np.arange(c.rows)
+    # Sequence 1's rows pushed again and again: `many` more tiles per head.
+    many = 256 // hk + 1
+    tiled = np.r_[alone, np.tile(np.flatnonzero(c.seq == 1), many)]
+    bits = []
+    for keep in (alone, both, tiled):
+        sub = W.PagedCase(hq=hq, hk=hk, page=c.page, pos=c.pos[keep], seq=c.seq[keep], ragged=1, indptr=c.indptr,
+                          pages=c.pages, num_pages=c.num_pages, qkv=c.qkv[keep], kv=c.kv)
+        pf = oa.prefill_plan(sub.rows, hq, hk, sub.page, sub.seq, sub.pos)
+        assert (pf.plan.tiles * hk > 256) == (keep is tiled) and pf.plan.tiles >= -(-rows // per)
+        bits.append(run_prefill(sub, exact_p=exact_p)[:rows])
+    assert np.array_equal(bits[0], bits[1]), f"{np.sum(bits[0] != bits[1])} elements differ beside another request"
+    assert np.array_equal(bits[0], bits[2]), f"{np.sum(bits[0] != bits[2])} elements differ in a large call"
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("hq,hk,q_len,kv_len", [(32, 8, 257, 334), (32, 8, 130, 900), (16, 8, 65, 64), (8, 8, 300, 300)])
+def test_dit_row_bits_do_not_depend_on_the_call(hq, hk, q_len, kv_len, causal):
+    """Without a workspace a problem's rows have the same bits alone (row halves),
+    as the first of a batch of one round of tiles (whole), and as the last of a
+    batch with a short last round (halved)."""
+    G, n = hq // hk, 256 // hk
+    tiles = -(-q_len * G // 256)
+    one = W.dense_case(hq, hk, q_len, kv_len, causal, seed=q_len)
+    want = run_dense(one)[0]
+    for batch in (-(-n // tiles), n // tiles + 1):
+        c = W.DenseCase(hq=hq, hk=hk, q_len=q_len, kv_len=kv_len, causal=causal, q_stride=one.q_stride,
+                        q=np.repeat(one.q, batch, 0), k=np.repeat(one.k, batch, 0), v=np.repeat(one.v, batch, 0),
+                        batch=batch)
+        got = run_dense(c)
+        for b in range(batch):
+            assert np.array_equal(got[b], want), f"batch {batch}, problem {b}: {np.sum(got[b] != want)} elements differ"
+
+
 @pytest.mark.parametrize("hq,hk,page", [(32, 8, 16), (16, 16, 16), (16, 8, 12), (64, 8, 16), (8, 4, 3)])
 def test_prefill_exact_p_parity(oracle, hq, hk, page):
     """The plan's exact_p (P carried as two bf16 terms through P.V) on every
