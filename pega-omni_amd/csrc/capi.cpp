@@ -543,7 +543,7 @@ int omni_hidream_attend_ws(const void* q, const void* k, const void* v, void* ou
   int items = 0;
   const int resident = resident_tiled_groups();
   omni::dit_split(a, batch, resident, &items, &a.split_from, &a.split_k);
-  if (items < resident) a.halved = omni::dit_halves(a, batch, resident);  // no split below a round
+  if (items < resident && a.split_k == 0) a.halved = omni::dit_halves(a, batch, resident);
   const int64_t need = (int64_t)(items - a.split_from) * a.split_k * omni::kSegmentBytes;
   if (need > workspace_bytes)
     return fail(OMNI_ATTN_EWORKSPACE, "hidream_attend: the split needs %lld workspace bytes, got %lld",

@@ -974,12 +974,19 @@ void dit_split(const TiledArgs& a, int batch, int resident, int* items, int* spl
   *items = (int)n;
   *split_from = (int)n;
   *split_k = 0;
-  // Calls of less than one round run as row parts within the launch instead
-  // (tiled_quarters, dit_halves): no partials in memory and no combine launch.
-  if (resident <= 0 || n < resident || n > (1LL << 30)) return;
+  if (resident <= 0 || n <= 0 || n > (1LL << 30)) return;
   const int rem = (int)(n % resident);
   if (rem == 0 || resident / rem < 2) return;
   const int chunks = std::min(resident / rem, std::max(2, (a.q_len + kBN - 1) / kBN / kMinChunkTiles));
+  // Calls of less than one round that would get only two or three chunks run as
+  // row parts within the launch instead (tiled_quarters, dit_halves): no partials
+  // in memory and no combine launch. us per call, by keys / by rows, 32q/8kv:
+  // 65 queries x 142 keys 14.7 / 8.0, 257 x 334 20.6 / 10.0, 257 x 4096 53.9 / 52.6,
+  // 1000 x 1077 37.3 / 23.5, 1024 x 4096 73.5 / 67.5 (past some 5000 keys for 257
+  // queries and 9000 for 1024 two chunks win again: 257 x 8192 92 / 100; the host
+  // does not know the key count). Four chunks, 4q/1kv, 4000 x 4000: 45.9 / 54.4;
+  // 8q/1kv, 2048 x 8192 72 / 103, 2048 x 2048 35.2 / 30.2.
+  if (n < resident && chunks < 4) return;
   *split_from = (int)n - rem;
   *split_k = chunks;
 }

@@ -408,6 +408,37 @@ def test_prefill_row_bits_do_not_depend_on_the_call(hq, hk, rows, cached, exact_
     assert np.array_equal(bits[0], bits[2]), f"{np.sum(bits[0] != bits[2])} elements differ in a large call"
 
 
+def splits_by_keys(hq, hk, q_len, batch=1):
+    """Whether hidream_attend_ws splits this shape by keys: a call with a
+    workspace of 16 bytes is refused exactly then."""
+    st = (hq + 2 * hk) * 128
+    q = torch.zeros(batch, q_len, st, dtype=torch.bfloat16, device="cuda")
+    k = torch.zeros(batch, 8, hk * 128, dtype=torch.bfloat16, device="cuda")
+    out = torch.zeros(batch, q_len, hq * 128, dtype=torch.bfloat16, device="cuda")
+    try:
+        oa.hidream_attend_ws(q, k, k, out, q_len, dev_i32(np.array([8], np.int32)), st, 0, 0.1, hq, hk, batch,
+                             q_len * st, 8 * hk * 128, q_len * hq * 128,
+                             torch.zeros(16, dtype=torch.uint8, device="cuda"))
+    except oa.OmniAttnError as e:
+        assert e.code == oa.EWORKSPACE
+        return True
+    finally:
+        torch.cuda.synchronize()
+    return False
+
+
+@pytest.mark.parametrize("hq,hk,q_len,batch,split", [
+    # below one round (256 CUs): by rows, unless at least four chunks of four key tiles fit
+    (32, 8, 65, 1, False), (32, 8, 1000, 1, False), (8, 1, 1920, 1, False), (8, 1, 1921, 1, True), (4, 1, 4000, 1, True),
+    (8, 2, 4000, 1, False),  # 126 items: two chunks
+    # past a round: the remainder, if at most half a round
+    (32, 8, 1100, 2, True), (32, 8, 2049, 1, True), (32, 8, 3000, 1, True), (32, 8, 3100, 1, False),
+])
+def test_dit_split_rule(hq, hk, q_len, batch, split):
+    """Which shapes a workspace call splits by keys."""
+    assert splits_by_keys(hq, hk, q_len, batch) == split
+
+
 @pytest.mark.parametrize("causal", [0, 1])
 @pytest.mark.parametrize("hq,hk,q_len,kv_len", [(32, 8, 257, 334), (32, 8, 130, 900), (16, 8, 65, 64), (8, 8, 300, 300)])
 def test_dit_row_bits_do_not_depend_on_the_call(hq, hk, q_len, kv_len, causal):
