@@ -80,12 +80,17 @@ int pick_chunk(int rows, int hq, int hk, int max_len) {
 
 // Split size for lm_attend over FP8 slots (decode_split_fp8, up to 8 heads per
 // workgroup): the largest of 1024 / 768 / 512 / 384 keys that still gives
-// >= 2048 workgroups of 8 heads at full length, else 256. Measured on MI355X
-// (PersonaPlex rows, lengths U[100, 3000], 32 heads, us per call): 32 rows
-// 99.7 / 87.9 / 84.9 / 79.7 / 79.7 at 1024 / 768 / 512 / 384 / 256; 64 rows
-// 143.7 / 135.5 / 130.1 / 130.9 / 136.2; 128 rows 294.2 / 275.6 / 276.7 /
-// 272.5 / 293.3; 256 rows 540.8 / 547.3 / 539.6 / 551.1 / 583.6. The bf16
-// rule above (1024 for all but the 32-row bucket) is 0-10% slower here.
+// >= 2048 workgroups of 8 heads at full length, else 256. PersonaPlex rows of 32
+// heads, fused call, lengths spread over 300-3000, us per layer at 1024 / 768 /
+// 512 / 384 / 256 keys, each at the heads per workgroup that the launch takes for
+// it (fp8_heads_per_group: 4, or 8 from 2048 workgroups of 8 at 512 keys on):
+// 16 rows 58.7 / 49.9 / 50.2 / 47.9 / 47.5; 32 rows 94.4 / 96.3 / 87.8 / 89.1 / 89.2;
+// 64 rows 175 / 167 / 150 / 150 / 158; 128 rows 291 / 297 / 290 / 293 / 306. (The line
+// was drawn at 8 heads throughout, lengths U[100, 3000], plain call: 32 rows 99.7 /
+// 87.9 / 84.9 / 79.7 / 79.7, 64 rows 143.7 / 135.5 / 130.1 / 130.9 / 136.2, 128 rows
+// 294.2 / 275.6 / 276.7 / 272.5 / 293.3, 256 rows 540.8 / 547.3 / 539.6 / 551.1 / 583.6;
+// both place it within 2.5% of the best split.) The bf16 rule above (1024 for all
+// but the 32-row bucket) is 0-10% slower here.
 int pick_chunk_fp8(int rows, int heads, int max_len) {
   for (int chunk : {1024, 768, 512, 384}) {
     const long long wgs = (long long)rows * ((heads + 7) / 8) * (((long long)max_len + chunk - 1) / chunk);

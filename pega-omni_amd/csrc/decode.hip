@@ -947,16 +947,25 @@ __global__ __launch_bounds__(64) void decode_combine(DecodeArgs a) {
 }
 
 // Heads per workgroup. Eight (1 KiB runs) for long splits that leave about 8
-// workgroups per CU; else four where they leave one per CU, two for a few
-// rows, one for a handful of short ones: a narrower group reads 128-byte runs
-// and loads its scales once per head, a wider one leaves CUs idle. Fused calls
-// of 32 heads, lengths from a tenth of max_len to max_len, the plan's splits,
-// us per layer at 1 / 2 / 4 / 8 heads:
-//   max_len 3000: 1 row 10.1 / 10.7 / 13.5 / 19.6, 5 rows 30.7 / 26.3 / 23.6 / 22.5,
-//     16 rows 69.1 / 52.1 / 48.6 / 46.7, 48 rows 191 / 138 / 123 / 128, 64 rows
-//     (384-key splits) 216 / 161 / 149 / 151, 128 rows (768-key splits) best at 8;
-//   max_len 400: 4 rows 10.4 / 10.9 / 14.1 / 19.3, 16 rows 20.3 / 15.7 / 15.3 / 20.8.
-// (Before: the widest group that leaves 2048 workgroups, so 1 head up to ten rows.)
+// workgroups per CU (256 CUs); else four where they leave one per CU, two for a
+// few rows, one for a handful of short ones: a narrower group reads 128-byte
+// runs and loads its scales once per head, a wider one leaves CUs idle. Fused
+// calls of 32 heads, lengths from a tenth of max_len to max_len, the FP8 plan's
+// splits (256 keys unless said), us per layer at 1 / 2 / 4 / 8 heads:
+//   max_len 3000: 2 rows 18.5 / 16.9 / 16.4 / 21.0, 5 rows 30.7 / 27.3 / 24.4 / 24.0,
+//     8 rows 43.1 / 35.1 / 33.0 / 36.7, 16 rows 68.9 / 51.5 / 47.8 / 47.4, 48 rows
+//     192 / 141 / 127 / 131, 64 rows (384 keys) 216 / 167 / 154 / 156, 128 rows (768
+//     keys) 366 / 300 / 293 / 297 (lengths U[100, 3000]: 281 / 275 at 4 / 8);
+//   max_len 1500: 3 rows 14.0 / 12.2 / 14.2 / 20.1, 6 rows 20.8 / 16.6 / 15.2 / 20.6,
+//     12 rows 31.0 / 25.6 / 24.0 / 23.5, 16 rows 42.5 / 32.6 / 30.7 / 33.6, 32 rows
+//     73.5 / 53.9 / 50.7 / 52.7;
+//   max_len 400: 4 rows 10.4 / 11.0 / 14.0 / 19.4, 8 rows 12.6 / 11.2 / 14.1 / 19.2,
+//     16 rows 20.5 / 15.5 / 15.3 / 20.8, 32 rows 34.2 / 24.5 / 21.8 / 21.9.
+// Not taken: eight heads at 256-key splits, 1-2% faster (plain calls up to 10%)
+// only where their groups number some 190 to 290, one round, and 4-11% slower at
+// 350 to 600. Rows far shorter than max_len leave most groups empty and favour
+// fewer heads: one row under max_len 3000 (192 groups of two) takes 10.2 / 10.7 at
+// one / two heads with 1650 keys and 14.0 / 11.9 with 3000.
 static int fp8_heads_per_group(const DecodeArgs& a, int rows) {
   if (a.group_heads) return a.group_heads;
   const auto groups = [&](int h) { return a.hk % h == 0 ? (int64_t)rows * (a.hk / h) * a.splits : 0; };
