@@ -207,7 +207,7 @@ typedef struct omni_attn_prefill_plan {
   int32_t tiles;     /* query tiles (each runs once per kv head) */
   int32_t tile_rows; /* packed (position, head) rows per tile */
   int64_t work_bytes; /* bytes of the int32 work list the caller uploads */
-  int32_t workgroups; /* grid of omni_attn_prefill_run */
+  int32_t workgroups; /* workgroups of a run that takes one per item (a run of few items takes two or four) */
   int32_t exact_p;    /* 0 (what plan_init sets): P rounded to bf16 for P.V, as the MFMA
                          flash kernels of the reference do (hidream.cu:317-324); 1: P carried
                          as two bf16 terms (hi + lo) through P.V, 16 significant bits, for
@@ -218,8 +218,11 @@ typedef struct omni_attn_prefill_plan {
 /* Host: validate (seq_h, pos_h) for `rows` ragged rows and write the work list
  * into work_h (capacity work_cap int32): a header of 16 int32 whose entries
  * 0..8 bound the item ranges of the GPU's 8 XCDs, then 4 int32 per (tile, kv
- * head) item (sequence, first row, rows, kv head). Workgroup i runs item
- * header[i % 8] + i / 8. In workgroup order the tiles run by the keys they
+ * head) item (sequence, first row, rows, kv head). Workgroup i takes item
+ * header[i % 8] + i / 8 if it is below header[i % 8 + 1]; where the items fill
+ * at most half (a quarter) of the GPU and the page is a multiple of 16, two
+ * (four) workgroups share an item's rows and i / 8 is i / 16 (i / 32). In
+ * workgroup order the tiles run by the keys they
  * see, most first, each with its hk kv heads, so every XCD ends on short
  * tiles and always sees the same kv heads (their K/V stays in its L2); the
  * XCD ranges differ by at most one item. Returns OMNI_ATTN_EWORKSPACE with plan->work_bytes set when
@@ -229,7 +232,8 @@ int omni_attn_prefill_plan_init(int rows, int hq, int hk, int page, const int32_
 
 /* Ragged causal prefill with the semantics of qwen3_attend(ragged = 1): row n
  * sees keys 0..pos[n] of sequence seq[n] through the page table. `work` is
- * the device copy of the plan's work list. */
+ * the device copy of the plan's work list. A row's bits depend on its own
+ * keys and position alone, not on the other rows or tiles of the call. */
 int omni_attn_prefill_run(const omni_attn_prefill_plan* plan, const void* qkv, const void* kv, const int32_t* pos,
                           const int32_t* seq, const int32_t* indptr, const int32_t* pages, void* out, float scale,
                           const int32_t* work, void* stream);
@@ -242,8 +246,9 @@ int omni_attn_prefill_run(const omni_attn_prefill_plan* plan, const void* qkv, c
  * only keys 0..n. A row that sees no key (*kv_len_at = 0) stores NaN, as the
  * reference's 1 / l does. The reference fixes G = 4 and hk = gridDim.y; here hq and hk
  * are arguments (G in {1,2,4,8}). When the last round of tiles would fill at
- * most half the GPU, its tiles run as two workgroups of half the rows each
- * (no workspace; each row is computed the same way). */
+ * most half the GPU, its tiles run as two workgroups of half the rows each, and
+ * a call of at most a quarter of the GPU as four per tile (no workspace; each
+ * row is computed the same way, to the same bits). */
 int omni_hidream_attend(const void* q, const void* k, const void* v, void* out, int q_len, const int32_t* kv_len_at,
                         int q_stride, int causal, float scale_log2, int hq, int hk, void* stream);
 

@@ -165,13 +165,22 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
   // DiT row halves: the last `halved` items, in the same order as the split
   // chunks.
   int idx, chunk = -1, part = -1;
+  int4 item{};  // prefill: sequence, first row, rows, kv head
   if constexpr (PAGED) {
-    // XCD x's range starts at header entry x, which the plan makes
-    // x (items / 8) + min(x, items % 8): computed, not read, so the item is
-    // the first load of the chain item -> sequence -> page ids -> K.
+    // XCD x's items are those from header entry x to entry x + 1. The plan puts
+    // its range at x (items / 8) + min(x, items % 8), so the item is read there
+    // beside the header, in one round trip, and once more only if the list's
+    // header says otherwise (the chain item -> sequence -> page ids -> K follows).
+    const auto at = [&](int i) {
+      const int32_t* it = a.work + kPrefillWorkHeader + 4 * (int64_t)i;
+      return int4{it[0], it[1], it[2], it[3]};
+    };
     const int x = blockIdx.x & 7, k = blockIdx.x >> 3, nth = k / PARTS;
-    if (nth >= (items >> 3) + (x < (items & 7))) return;
-    idx = x * (items >> 3) + min(x, items & 7) + nth;
+    idx = min(x * (items >> 3) + min(x, items & 7) + nth, items - 1);
+    item = at(idx);
+    const int first = a.work[x] + nth;
+    if (first >= a.work[x + 1]) return;
+    if (first != idx) item = at(idx = first);
     if constexpr (PARTS > 1) part = PARTS - 1 - k % PARTS;  // a tile's later rows see more keys
   } else if constexpr (FORM == kHalves) {
     const int halves_from = items - a.halved;
@@ -213,9 +222,8 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       idx /= PARTS;
     }
   }
-  const int32_t* item = PAGED ? a.work + kPrefillWorkHeader + 4 * idx : nullptr;
   const int tile = PAGED ? 0 : idx % ntiles;
-  const int kvh = PAGED ? item[3] : (idx / ntiles) % a.hk;
+  const int kvh = PAGED ? item.w : (idx / ntiles) % a.hk;
   const int b = PAGED ? 0 : idx / (ntiles * a.hk);
   constexpr int kPos = kBM / G;  // positions per tile
   constexpr int kPartPos = kPos / PARTS;  // and per part
@@ -226,8 +234,8 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
 
   Tile t;
   if constexpr (PAGED) {
-    const int s = item[0], first = item[1];
-    t.nq = item[2];
+    const int s = item.x, first = item.y;
+    t.nq = item.z;
     if (no_rows(t.nq)) return;
     t.pos = a.pos + first;
     t.q = a.q + (int64_t)first * a.q_stride;

@@ -385,6 +385,40 @@ def test_dit_workgroups_per_tile(oracle, q_len, kv_len, batch, causal):
         assert_close(whole[-1][pick], want, what="picked rows")
 
 
+@pytest.mark.parametrize("new", [100, 300, 900])  # 32, 80 and 240 items: quarters, halves, whole tiles
+@pytest.mark.parametrize("page", [16, 12])
+def test_prefill_item_ranges_follow_the_lists_header(new, page):
+    """The work list's header bounds the items that run: ranges moved between
+    XCDs run the same items, and an item left out of them stays unwritten."""
+    c = W.ragged_prefill_case(2, 32, 8, new, new, 0, 100, page=page, seed=new)
+    pf = oa.prefill_plan(c.rows, 32, 8, page, c.seq, c.pos)
+    head, items = pf.work[:9].cpu().numpy(), pf.plan.tiles * 8
+    assert head[0] == 0 and head[8] == items and pf.plan.workgroups == items  # ranges of items / 8 each
+
+    def run(header):
+        out = torch.zeros(c.rows, 32 * 128, dtype=torch.bfloat16, device="cuda")
+        work = pf.work.clone()
+        work[:9] = dev_i32(header)
+        oa.prefill_run(oa.Prefill(pf.plan, work), dev_bits(c.qkv), dev_bits(c.kv), dev_i32(c.pos), dev_i32(c.seq),
+                       dev_i32(c.indptr), dev_i32(c.pages), out, c.scale)
+        torch.cuda.synchronize()
+        return host_bits(out)
+
+    whole = run(head)
+    body = pf.work[16:].view(-1, 4).cpu().numpy()
+    cut = head.copy()
+    cut[8] -= 1  # the last item is in no range
+    got, (_, first, n, h) = run(cut), body[items - 1]
+    left = np.zeros((c.rows, 32, 128), bool)
+    left[first:first + n, 4 * h:4 * h + 4] = True
+    left = left.reshape(c.rows, -1)
+    assert np.array_equal(got[~left], whole[~left]) and not got[left].any() and whole[left].any()
+    moved = head.copy()
+    moved[1:8] -= 1  # range 0 loses its last item, 1..6 begin one earlier, 7's last item is left out
+    moved[8] -= 1
+    assert np.array_equal(run(moved), got)
+
+
 @pytest.mark.parametrize("exact_p", [False, True])
 @pytest.mark.parametrize("hq,hk,rows,cached", [(16, 8, 187, 0), (32, 8, 150, 700), (16, 16, 40, 300), (64, 8, 33, 1000)])
 def test_prefill_row_bits_do_not_depend_on_the_call(hq, hk, rows, cached, exact_p):
