@@ -106,6 +106,12 @@ __device__ __forceinline__ bf16x4 lds_read_tr(const bf16_t* p) {
 
 __device__ __forceinline__ bf16x8 as_bf16x8(const uint4& u) { return __builtin_bit_cast(bf16x8, u); }
 
+// Orders a wave's LDS writes before its own later LDS reads of other lanes' data.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // Pack 8 f32 to 8 bf16 (RNE) as an MFMA operand.
 __device__ __forceinline__ bf16x8 pack8(const float* v) {
   uint4 u;
@@ -792,6 +798,9 @@ __global__ __launch_bounds__(kThreads, 1) void tiled_attn(TiledArgs a, int items
       w.y = pack_bf16x2(o[md][4 * q4 + 2] * inv, o[md][4 * q4 + 3] * inv);
       *reinterpret_cast<uint2*>(rows + jn * kHead + 8 * ((4 * md + q4) ^ (jn & 15)) + 4 * hn) = w;
     }
+  // Lanes read what other lanes of the wave wrote: LDS keeps a wave's accesses in
+  // order, and this keeps the compiler's.
+  wave_lds_fence();
   // The block's rows, four per instruction, a 16-byte chunk per lane.
 #pragma unroll
   for (int i = 0; i < 8; ++i) {

@@ -68,3 +68,18 @@ def test_the_checker_catches_a_missing_wait():
     bad = 'asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" : : "v"(x), "s"(r), "{m0}"(l) : "memory");'
     (line, template, operands, prev), = asm_blocks(bad)
     assert VMEM.search(template) and re.search(r'"s"', operands) and not SNOP.match(template)
+
+
+def test_rows_exchanged_through_lds_are_fenced():
+    """The output rows of the tiled kernels go through LDS: a lane reads 16-byte
+    chunks that other lanes wrote in 8-byte halves. Between such a write and the
+    read after it stands a barrier or the wave fence; without one nothing tells
+    the compiler that the two may not trade places."""
+    text = open(os.path.join(CSRC, "tiled.hip")).read()
+    writes = [m.start() for m in re.finditer(r"\*reinterpret_cast<uint2\*>\(rows \+", text)]
+    reads = [m.start() for m in re.finditer(r"\*reinterpret_cast<const uint4\*>\(rows \+", text)]
+    assert len(writes) == len(reads) == 2  # whole tiles and halves, quarters
+    for w, r in zip(writes, reads):
+        assert w < r and re.search(r"wave_lds_fence\(\);|__syncthreads\(\);", text[w:r])
+    body = re.search(r"void wave_lds_fence\(\) \{(.*?)\n\}", text, flags=re.S).group(1)
+    assert "__builtin_amdgcn_fence(__ATOMIC_ACQ_REL" in body and "__builtin_amdgcn_wave_barrier()" in body
