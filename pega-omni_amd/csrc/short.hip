@@ -192,9 +192,10 @@ __global__ __launch_bounds__(64 * kMimiWaves) void mimi_attend64(ShortArgs a) {
 #pragma unroll
     for (int j = TR - 1; j >= 0; --j) {
       if (tb >= len[j]) continue;
-      // A slot that only a later row of the session sees: its p is 0 here, and
-      // its V row must not reach the sum (0 times an infinity would).
-      if (len[j] < slots) {
+      // A lane past the row's slots (one that only a later row of the session
+      // sees, or past the last): its p is 0 here, and the V row it holds must not
+      // reach the sum (0 times an infinity would).
+      if (tb + R * NI > len[j]) {
 #pragma unroll
         for (int i = 0; i < NI; ++i)
           if (tb + R * i + r >= len[j]) vr[i] = uint4{};

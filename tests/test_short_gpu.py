@@ -96,6 +96,31 @@ def test_mimi_attend_slots_of_infinite_keys(oracle, first, count):
     assert_close(host_bits(out), want, what="mimi_attend")
 
 
+@pytest.mark.parametrize("T", [1, 2])
+@pytest.mark.parametrize("wrapped", [False, True])
+def test_mimi_attend_infinite_v_in_the_last_slot(oracle, T, wrapped):
+    """An infinite V in the ring's last slot: every row that sees it gives
+    infinities, not NaN (the lanes past the last slot weigh 0 and must not
+    multiply its V); rows before it stay finite."""
+    c = mimi_case(11, sessions=3, T=T, heads=3, context=250)
+    c["pos"][:] = 400 // T if wrapped else 248 // T  # a last slot off a trip's end either way (249 or 248)
+    slot = 2 * 3 * 64
+    last = 249 if wrapped else 248 // T * T + T - 1
+    for line in c["lines"]:
+        at = int(line) * c["stride"] // 2 + last * slot + slot // 2
+        c["state"].view(np.uint16)[at:at + slot // 2] = 0x7F80
+    args = (c["lines"], c["state"], c["rows"], T, 3, 0.125, 250, c["stride"])
+    want = oracle.mimi_attend(c["qkv"], c["pos"], *args)
+    out = torch.zeros(c["rows"], 3 * 64, dtype=torch.bfloat16, device="cuda")
+    oa.mimi_attend(dev_bits(c["qkv"]), dev_i32(c["pos"]), dev_i32(c["lines"]), torch.from_numpy(c["state"]).cuda(), out,
+                   c["rows"], T, 3, 0.125, 250, c["stride"])
+    torch.cuda.synchronize()
+    got, inf = host_bits(out), want == 0x7F80
+    assert inf.any() and np.array_equal(got == 0x7F80, inf)
+    if not inf.all():
+        assert_close(got[~inf], want[~inf], what="mimi_attend")
+
+
 @pytest.mark.parametrize("seed,sessions,heads,pos_hi", [(4, 4, 4, 200), (5, 64, 16, 1000), (6, 3, 2, 3)])
 def test_codec_attention(oracle, seed, sessions, heads, pos_hi):
     c = codec_case(seed, sessions=sessions, heads=heads, pos_hi=pos_hi)
