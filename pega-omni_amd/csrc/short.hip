@@ -152,12 +152,26 @@ struct Row64 {
 // 8 x 4 61 / 80 / 180, 4 x 8 64 / 83 / 196 us (more loads per trip cost
 // registers, and so occupancy); one row per workgroup 58-60 / 91-95 / 199-209;
 // two heads per workgroup (256-byte runs) 71 / 85 / 153 us.
+//
+// Few workgroups take one row each (kMimiAlone): a pair's code is twice as long
+// and its call 0.6 us longer at the least, and CUs that would idle read the K and
+// V rows again. us per layer, pairs / single rows, 8 heads, T = 2, positions
+// 3-400 (0-7): 1 session 3.25 / 2.67 (3.23 / 2.63), 8 5.6 / 4.8 (3.35 / 2.82), 16
+// (256 workgroups) 5.8 / 5.3 (3.56 / 2.83), 24 6.1 / 6.7 (3.7 / 3.0), 32 6.3 / 7.7
+// (3.7 / 3.0), 128 14.2 / 20.0 (7.1 / 4.9).
+// A context of at most one wave's slots takes one wave: context 8, 32 sessions
+// 3.65 -> 2.68, 128 6.97 -> 3.79. One wave per (row, head) throughout would take
+// 3.0 and 3.8 us for 32 and 128 sessions that are all at positions 0-7, where
+// pairs take 3.7 and 7.1, but 13.4 and 20.8 at positions 3-400, and a call lasts
+// as long as its longest ring. (Ending the waves that have no slots at once: 128
+// sessions at 0-7 5.2, all other calls 3-5% longer.)
 constexpr int kMimiWaves = 8;
 constexpr int kMimiLoads = 2;
+constexpr int kMimiAlone = 256;  // workgroups of one row: one per CU
 
-template <int TR>
-__global__ __launch_bounds__(64 * kMimiWaves) void mimi_attend64(ShortArgs a) {
-  constexpr int W = kMimiWaves, NI = kMimiLoads, R = 8;  // R slots per load instruction
+template <int TR, int W = kMimiWaves>
+__global__ __launch_bounds__(64 * W) void mimi_attend64(ShortArgs a) {
+  constexpr int NI = kMimiLoads, R = 8;  // R slots per load instruction
   const int n0 = blockIdx.x * TR, h = blockIdx.y;
   const int lane = threadIdx.x & 63, c = lane & 7, r = lane >> 3;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -411,8 +425,10 @@ int launch_short(const ShortArgs& a, int kind, hipStream_t stream) {
   if (a.rows == 0) return 0;
   const dim3 grid(a.rows, a.heads);
   switch (kind) {
-    case kShortMimi:  // an even T: a session's rows in pairs
-      if (a.T % 2 == 0)
+    case kShortMimi:  // an even T: a session's rows in pairs, unless the call is small
+      if (a.context <= 8 * kMimiLoads)
+        mimi_attend64<1, 1><<<grid, 64, 0, stream>>>(a);
+      else if (a.T % 2 == 0 && (int64_t)a.rows * a.heads > kMimiAlone)
         mimi_attend64<2><<<dim3((a.rows + 1) / 2, a.heads), 64 * kMimiWaves, 0, stream>>>(a);
       else
         mimi_attend64<1><<<grid, 64 * kMimiWaves, 0, stream>>>(a);

@@ -121,6 +121,28 @@ def test_mimi_attend_infinite_v_in_the_last_slot(oracle, T, wrapped):
         assert_close(got[~inf], want[~inf], what="mimi_attend")
 
 
+@pytest.mark.parametrize("T", [2, 4])
+@pytest.mark.parametrize("context", [16, 17, 250])  # one wave per row; eight
+def test_mimi_attend_either_side_of_its_launches(oracle, T, context):
+    """Sessions up to one workgroup per CU (256 row x head pairs: rows alone) and
+    one session more (rows in pairs) against the oracle; a session's bits are
+    the same in both."""
+    heads, n = 8, 256 // 8 // T
+    c = mimi_case(12, sessions=n + 1, T=T, heads=heads, context=context)
+    c["pos"] = np.linspace(0, 300 // T, n + 1).astype(np.int32)
+    want = oracle.mimi_attend(c["qkv"], c["pos"], c["lines"], c["state"], c["rows"], T, heads, 0.125, context,
+                              c["stride"])
+    state, got = torch.from_numpy(c["state"]).cuda(), []
+    for rows in (n * T, (n + 1) * T):
+        out = torch.zeros(rows, heads * 64, dtype=torch.bfloat16, device="cuda")
+        oa.mimi_attend(dev_bits(c["qkv"]), dev_i32(c["pos"]), dev_i32(c["lines"]), state, out, rows, T, heads, 0.125,
+                       context, c["stride"])
+        torch.cuda.synchronize()
+        got.append(host_bits(out))
+        assert_close(got[-1], want[:rows], what="mimi_attend")
+    assert np.array_equal(got[0], got[1][:n * T])
+
+
 @pytest.mark.parametrize("seed,sessions,heads,pos_hi", [(4, 4, 4, 200), (5, 64, 16, 1000), (6, 3, 2, 3)])
 def test_codec_attention(oracle, seed, sessions, heads, pos_hi):
     c = codec_case(seed, sessions=sessions, heads=heads, pos_hi=pos_hi)
