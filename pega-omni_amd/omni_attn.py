@@ -180,14 +180,20 @@ def _check(rc: int):
 # layer: 13 us of host against 11 us of kernels), so the checks below read each
 # attribute once, pointers go to ctypes as plain integers (every pointer
 # parameter is declared c_void_p) and the stream is asked for as a raw handle
-# instead of a torch.cuda.Stream object.
+# instead of a torch.cuda.Stream object (torch's own call for it is not a public
+# one: where a build lacks it, the public one answers).
+_raw_stream = getattr(_torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
 def _stream(stream):
     if stream is None:
-        return _torch._C._cuda_getCurrentRawStream(_torch.cuda.current_device())
+        if _raw_stream is not None:
+            return _raw_stream(_torch.cuda.current_device())
+        stream = _torch.cuda.current_stream()
     return stream.cuda_stream
 
 

@@ -414,3 +414,16 @@ def test_mimi_rope_kv_and_copy_kv_validate_before_launch():
     assert L.omni_lm_copy_kv(f, f, f, -1, 8448, None) == oa.EINVAL
     assert L.omni_lm_copy_kv(odd, f, f, 3, 8448, None) == oa.EINVAL
     assert L.omni_lm_copy_kv(f, None, f, 3, 8448, None) == oa.EINVAL
+
+
+@pytest.mark.parametrize("raw", [True, False])
+def test_the_current_streams_handle(monkeypatch, raw):
+    """No stream given: the current stream of the current device, by torch's raw
+    handle where the build has that call and by torch.cuda.current_stream where not."""
+    class Stream:
+        cuda_stream = 0x77
+    monkeypatch.setattr(oa, "_raw_stream", (lambda dev: 0x70 + dev) if raw else None)
+    monkeypatch.setattr(oa._torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(oa._torch.cuda, "current_stream", Stream)
+    assert oa._stream(None) == (0x73 if raw else 0x77)
+    assert oa._stream(Stream()) == 0x77
