@@ -110,15 +110,30 @@ def oracle_dense(oracle, c, b=0, kv_len=None):
                                c.causal, c.scale_log2, nthreads=16)
 
 
-# On a 256-CU GPU the workspace-free call runs the last round's items as row
-# halves when they fill at most half of it: every case below but the
-# 1100-query one (144 items, all whole) runs as halves only. (16, 8, 65) and
-# (4, 4, 1) have second halves with one and no rows.
-@pytest.mark.parametrize("hq,hk,q_len,kv_len,causal", [
-    (32, 8, 300, 300, 1), (32, 8, 257, 333, 0), (8, 8, 100, 130, 0), (4, 4, 1, 1, 0), (16, 8, 65, 64, 1),
-    (32, 4, 40, 500, 0), (32, 8, 1100, 300, 1),
+def dit_path(hq, hk, q_len, batch=1, ws=False):
+    """How a DiT call runs its 256-row tiles (a mirror of the library's rule):
+    whole; all as row quarters; those past whole rounds as row halves, or, with a
+    workspace, as (count of) key chunks."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    items = -(-q_len // (256 * hk // hq)) * hk * batch
+    rem = items % cus
+    if ws and 0 < rem <= cus // 2:
+        chunks = min(cus // rem, max(2, -(-q_len // 128) // 4))
+        if items >= cus or chunks >= 4:
+            return f"{chunks} chunks"
+    return "quarters" if items * 4 <= cus else "halves" if 0 < rem <= cus // 2 else "whole"
+
+
+# On 256 CUs. (16, 8, 65) and (4, 4, 1) have quarters with few and no rows, (8, 8,
+# 2049) and (32, 4, 520) last tiles of a few rows.
+@pytest.mark.parametrize("hq,hk,q_len,kv_len,causal,path", [
+    (32, 8, 300, 300, 1, "quarters"), (32, 8, 257, 333, 0, "quarters"), (8, 8, 100, 130, 0, "quarters"),
+    (4, 4, 1, 1, 0, "quarters"), (16, 8, 65, 64, 1, "quarters"), (32, 4, 40, 500, 0, "quarters"),
+    (8, 8, 2049, 400, 1, "halves"), (16, 8, 1100, 300, 0, "halves"), (32, 8, 600, 520, 1, "halves"),
+    (32, 4, 520, 200, 0, "halves"), (32, 8, 1100, 300, 1, "whole"), (16, 16, 2200, 150, 0, "whole"),
 ])
-def test_dit_parity(oracle, hq, hk, q_len, kv_len, causal):
+def test_dit_parity(oracle, hq, hk, q_len, kv_len, causal, path):
+    assert dit_path(hq, hk, q_len) == path
     c = W.dense_case(hq, hk, q_len, kv_len, causal, seed=q_len)
     assert_close(run_dense(c)[0], oracle_dense(oracle, c), what=f"dit {hq}/{hk} {q_len}x{kv_len} c{causal}")
 
@@ -162,17 +177,44 @@ def run_dense_ws(c, kv_len=None):
 
 
 @pytest.mark.parametrize("hq,hk,q_len,kv_len,causal,batch", [
-    # (with 256-row tiles, 128-key tiles and 256 resident workgroups on MI355X)
-    (8, 2, 256, 256, 0, 1),     # 8 items, each split into 32 chunks of a 2-tile key range (most chunks empty)
-    (32, 8, 300, 700, 1, 2),    # causal: chunk ranges differ per tile
-    (32, 8, 1000, 1000, 0, 1),  # 128 items: each split in two
-    (4, 4, 1, 1, 0, 1),
+    (8, 2, 256, 256, 0, 1), (32, 8, 300, 700, 1, 2), (32, 8, 1000, 1000, 0, 1), (4, 4, 1, 1, 0, 1),
 ])
-def test_dit_tail_split_parity(oracle, hq, hk, q_len, kv_len, causal, batch):
+def test_dit_small_calls_with_a_workspace(oracle, hq, hk, q_len, kv_len, causal, batch):
+    """Calls of less than a round (8, 80, 128 and 4 tiles) that could be split in
+    fewer than four chunks: the workspace stays unused."""
+    assert dit_path(hq, hk, q_len, batch, ws=True) == dit_path(hq, hk, q_len, batch)
     c = W.dense_case(hq, hk, q_len, kv_len, causal, batch=batch, seed=q_len + kv_len)
     got = run_dense_ws(c)
     for b in range(batch):
         assert_close(got[b], oracle_dense(oracle, c, b), what=f"ws dit {hq}/{hk} {q_len}x{kv_len} c{causal} b{b}")
+
+
+# Every G, with more chunks than key tiles in some (chunks without a key).
+SPLITS = [
+    (8, 8, 8200, 300, 1, 16),    # 264 tiles, the last 8 split; 3 key tiles
+    (16, 8, 4100, 700, 1, 8),    # 264; 6 key tiles
+    (32, 8, 2049, 130, 1, 4),    # 264; 2 key tiles, the last query tile one position
+    (32, 8, 1100, 1500, 2, 2),   # 288
+    (32, 4, 2060, 520, 1, 4),    # 260; 5 key tiles
+    (32, 32, 257, 300, 5, 2),    # 320
+    (8, 1, 1921, 1000, 1, 4),    # 61 tiles, all split
+]
+
+
+@pytest.mark.parametrize("causal", [0, 1])
+@pytest.mark.parametrize("hq,hk,q_len,kv_len,batch,chunks", SPLITS)
+def test_dit_tail_split_parity(oracle, hq, hk, q_len, kv_len, batch, chunks, causal):
+    """Tiles past whole rounds as key chunks with a workspace and as row halves
+    (61 tiles: quarters) without one: every row of the first and last problem
+    against the oracle in both forms."""
+    assert dit_path(hq, hk, q_len, batch, ws=True) == f"{chunks} chunks" and splits_by_keys(hq, hk, q_len, batch)
+    assert dit_path(hq, hk, q_len, batch) == ("quarters" if hk == 1 else "halves")
+    c = W.dense_case(hq, hk, q_len, kv_len, causal, batch=batch, seed=q_len + kv_len)
+    split, rows = run_dense_ws(c), run_dense(c)
+    for b in {0, batch - 1}:
+        want = oracle_dense(oracle, c, b)
+        assert_close(split[b], want, what=f"chunks {hq}/{hk} {q_len}x{kv_len} c{causal} b{b}")
+        assert_close(rows[b], want, what=f"row parts {hq}/{hk} {q_len}x{kv_len} c{causal} b{b}")
 
 
 @pytest.mark.parametrize("hk,seed", [(8, 5000), (32, 5032)])
@@ -211,12 +253,18 @@ def test_dit_row_halves_match_split(oracle, causal):
 
 
 @pytest.mark.parametrize("causal", [0, 1])
-def test_dit_no_key_gives_nan(oracle, causal):
+@pytest.mark.parametrize("q_len,paths", [
+    (65, ("quarters", "quarters", "quarters")), (300, ("quarters", "halves", "halves")),
+    (1100, ("whole", "halves", "2 chunks")), (2049, ("halves", "halves", "4 chunks")),
+])
+def test_dit_no_key_gives_nan(oracle, causal, q_len, paths):
     """*kv_len_at = 0 (hidream.cu:337-346: l = 0, so O * (1 / l) = NaN): every
-    output element is NaN through the plain call, the batched call (row halves
-    for the last round) and the workspace call (key chunks, all empty), as the
-    oracle gives; a second call with keys overwrites them with finite values."""
-    c = W.dense_case(32, 8, 300, 300, causal, batch=2, seed=41 + causal)
+    output element is NaN through the plain call, the batched call and the
+    workspace call (key chunks, all empty), each running its tiles as `paths`
+    says, as the oracle gives; a second call with keys overwrites them with
+    finite values."""
+    assert (dit_path(32, 8, q_len), dit_path(32, 8, q_len, 2), dit_path(32, 8, q_len, 2, ws=True)) == paths
+    c = W.dense_case(32, 8, q_len, 300, causal, batch=2, seed=41 + causal)
     want = oracle.dense_attend(np.ascontiguousarray(c.q[0]), np.ascontiguousarray(c.k[0]), np.ascontiguousarray(c.v[0]),
                                c.q_len, 0, c.q_stride, c.hq, c.hk, causal, c.scale_log2, nthreads=16)
     assert np.isnan(bits_to_f64(want)).all()
@@ -355,34 +403,16 @@ def test_prefill_workgroups_per_tile(oracle, rows, cached, hq, hk, exact_p):
 
 
 @pytest.mark.parametrize("causal", [0, 1])
-@pytest.mark.parametrize("q_len,kv_len,batch", [
-    (16, 40, 1), (513, 600, 1), (1024, 1000, 1), (1025, 1102, 1), (520, 520, 2),  # 4, 2, 2, 1, 1 workgroups per tile
-    (1100, 1024, 2),  # 288 items: 32 past a round, split by keys with a workspace, as row halves without
+@pytest.mark.parametrize("q_len,kv_len,batch,path", [
+    (16, 40, 1, "quarters"), (512, 700, 1, "quarters"), (513, 600, 1, "halves"), (1024, 1000, 1, "halves"),
+    (1025, 1102, 1, "whole"), (520, 520, 2, "whole"), (1100, 1024, 2, "halves"),
 ])
-def test_dit_workgroups_per_tile(oracle, q_len, kv_len, batch, causal):
-    """DiT calls either side of each choice, with and without a workspace,
-    against the oracle on up to 64 rows of the last problem."""
+def test_dit_workgroups_per_tile(oracle, q_len, kv_len, batch, path, causal):
+    """DiT calls either side of each choice (64 and 72 tiles, 128 and 136, 144, 288
+    = a round and 32) against the oracle on every row of the last problem."""
+    assert dit_path(32, 8, q_len, batch) == path
     c = W.dense_case(32, 8, q_len, kv_len, causal, batch=batch, seed=q_len + kv_len)
-    whole, ws = run_dense(c), run_dense_ws(c)
-    assert_close(ws, whole, what="workspace vs none")
-    if causal:
-        n = min(64, q_len)
-        want = oracle.dense_attend(np.ascontiguousarray(c.q[-1, :n]), np.ascontiguousarray(c.k[-1]),
-                                   np.ascontiguousarray(c.v[-1]), n, kv_len, c.q_stride, 32, 8, 1, c.scale_log2,
-                                   nthreads=16)
-        assert_close(whole[-1][:n], want, what="first rows, causal")
-        if q_len > kv_len:  # rows past the keys see all of them
-            n = q_len - kv_len
-            want = oracle.dense_attend(np.ascontiguousarray(c.q[-1, -n:]), np.ascontiguousarray(c.k[-1]),
-                                       np.ascontiguousarray(c.v[-1]), n, kv_len, c.q_stride, 32, 8, 0, c.scale_log2,
-                                       nthreads=16)
-            assert_close(whole[-1][-n:], want, what="last rows, causal")
-    else:
-        pick = np.unique(np.r_[0, q_len - 1, np.linspace(0, q_len - 1, 62).astype(int)])
-        want = oracle.dense_attend(np.ascontiguousarray(c.q[-1, pick]), np.ascontiguousarray(c.k[-1]),
-                                   np.ascontiguousarray(c.v[-1]), len(pick), kv_len, c.q_stride, 32, 8, 0,
-                                   c.scale_log2, nthreads=16)
-        assert_close(whole[-1][pick], want, what="picked rows")
+    assert_close(run_dense(c)[-1], oracle_dense(oracle, c, batch - 1), what=f"{q_len}x{kv_len} c{causal}")
 
 
 @pytest.mark.parametrize("new", [100, 300, 900])  # 32, 80 and 240 items: quarters, halves, whole tiles
