@@ -965,7 +965,10 @@ __global__ __launch_bounds__(64) void decode_combine(DecodeArgs a) {
 // only where their groups number some 190 to 290, one round, and 4-11% slower at
 // 350 to 600. Rows far shorter than max_len leave most groups empty and favour
 // fewer heads: one row under max_len 3000 (192 groups of two) takes 10.2 / 10.7 at
-// one / two heads with 1650 keys and 14.0 / 11.9 with 3000.
+// one / two heads with 1650 keys and 14.0 / 11.9 with 3000. Against the widest
+// group that leaves 2048 workgroups (one head up to ten rows) that costs two and
+// three rows 3-7%: 2 rows of 300 and 3000 keys 14.6 -> 15.0 (plain 13.8 -> 14.8), 3
+// rows of 90-900 11.8 -> 12.4, for the gains of 6-45 rows (9 of 300-3000 43.2 -> 30.2).
 static int fp8_heads_per_group(const DecodeArgs& a, int rows) {
   if (a.group_heads) return a.group_heads;
   const auto groups = [&](int h) { return a.hk % h == 0 ? (int64_t)rows * (a.hk / h) * a.splits : 0; };
