@@ -59,17 +59,25 @@ int resident_tiled_groups() {
 //   CU: no partials and no combine. 512 against 256 keys: 32 rows 12.5 / 14.9,
 //   64 rows 20.3 / 22.3, 96 rows 25.6 / 29.2, 32 MHA rows 27.6 / 36.5.
 // - few workgroups: 128 keys, so that a wave has one tile and the keys spread
-//   over more CUs, while all of them still run at once: up to 512, or 256 for
-//   MHA, whose kernel holds two register tiles, and for rows of more than eight
-//   such splits, whose merge grows. 128 against 256 keys: 4 rows of up
-//   to 512 keys 7.9 / 9.6, 1 row of 2400 7.7 / 9.8, 8 of 1000 10.2 / 10.6, 2 MHA
-//   rows of 400 (hk = 32) 8.8 / 9.7; past it, fused with the rotary, 8 rows of 32q/8kv
-//   518-2468 (1280 workgroups) 26.4 / 21.6, 3 MHA rows of 1139-1544 (hk = 16, 624)
-//   19.1 / 17.1, 3 rows of 1364-1621 (312, 13 splits) 11.5 / 10.9.
+//   over more CUs, where that takes no more rounds of one workgroup per CU than
+//   256 keys do (one, or two where 256 keys take two too; MHA, whose kernel holds
+//   two register tiles, and rows of more than eight such splits: one). 128 against
+//   256 keys: 4 rows of up to 512 keys 7.9 / 9.6, 1 row of 2400 7.7 / 9.8, 2 MHA
+//   rows of 400 (hk = 32) 8.8 / 9.7; in two rounds both, 18 rows of 378 11.1 / 13.5
+//   (32q/8kv 13.5 / 16.5). A round more gains little on long rows and loses on
+//   short ones, whose workgroups without keys come first: plan for 8 rows of 1000,
+//   all of 1000 keys 12.0 / 12.3, 125-1000 10.5 / 10.9, all of 250 9.8 / 9.0, all
+//   of 125 8.5 / 7.0 (32q/8kv 14.1 / 14.6, 12.8 / 13.4, 12.2 / 11.6, 10.9 / 8.8).
+//   And not past 32 splits (48 for G = 4, whose tiles take longest): the merge
+//   grows. 1 row, hk = 1, of 4096 / 6000 / 8000 / 16000 keys: G = 1 10.1 / 10.2,
+//   11.2 / 10.3, 12.7 / 10.9, 17.6 / 14.0; G = 4 11.5 / 13.1, 12.7 / 13.4, 14.3 /
+//   14.2, 19.1 / 17.1.
 int pick_chunk(int rows, int hq, int hk, int max_len) {
   const long long units = (long long)rows * hk;
   if (max_len > 256 && max_len <= 512 && units >= 256) return 512;
-  if (max_len > 256 && units * (((long long)max_len + 127) / 128) <= (hq == hk || max_len > 1024 ? 256 : 512)) return 128;
+  const long long w128 = units * (((long long)max_len + 127) / 128), w256 = units * (((long long)max_len + 255) / 256);
+  const bool two_rounds = hq != hk && max_len <= 1024 && w256 > 256 && w128 <= 512;
+  if (max_len > 256 && max_len <= (hq == 4 * hk ? 6144 : 4096) && (w128 <= 256 || two_rounds)) return 128;
   int chunk = 1024;
   while (chunk > 256) {
     if (units * (((long long)max_len + chunk - 1) / chunk) >= 4096) break;

@@ -42,15 +42,22 @@ def test_decode_plan_shapes():
 
 
 @pytest.mark.parametrize("rows,hq,hk,max_len,chunk", [
-    (4, 16, 8, 256, 256), (4, 16, 8, 257, 128), (16, 16, 8, 512, 128), (17, 16, 8, 512, 256), (32, 16, 8, 512, 512),
-    (32, 16, 8, 513, 256), (512, 16, 8, 513, 1024), (8, 32, 8, 1024, 128), (4, 32, 8, 1025, 256),
-    (3, 16, 8, 1280, 128), (3, 16, 8, 1281, 256), (1, 16, 8, 4096, 128), (1, 16, 8, 4097, 256),
+    (4, 16, 8, 256, 256), (4, 16, 8, 257, 128), (8, 16, 8, 512, 128), (9, 16, 8, 512, 256), (17, 16, 8, 512, 256),
+    (32, 16, 8, 512, 512), (32, 16, 8, 513, 256), (512, 16, 8, 513, 1024), (4, 32, 8, 1024, 128), (5, 32, 8, 1024, 256),
+    (8, 32, 8, 1024, 256), (4, 32, 8, 1025, 256), (3, 16, 8, 1280, 128), (3, 16, 8, 1281, 256),
+    # in two rounds where 256-key splits take two as well
+    (10, 16, 8, 384, 128), (11, 16, 8, 384, 256), (16, 16, 8, 384, 256), (17, 16, 8, 384, 128), (21, 16, 8, 384, 128),
+    (22, 16, 8, 384, 256), (17, 16, 16, 384, 512), (9, 32, 32, 300, 512), (6, 32, 32, 300, 256),
+    # at most 32 splits of one row, 48 where four query heads share a K/V head
+    (1, 16, 8, 4096, 128), (1, 16, 8, 4097, 256), (1, 2, 1, 4096, 128), (1, 2, 1, 4097, 256), (1, 1, 1, 4097, 256),
+    (1, 4, 1, 6144, 128), (1, 4, 1, 6145, 256), (1, 4, 1, 32768, 256),
     (2, 32, 32, 512, 128), (2, 32, 32, 513, 256), (7, 32, 32, 512, 256), (8, 32, 32, 512, 512), (64, 16, 8, 2400, 256),
 ])
 def test_decode_plan_short_launches(rows, hq, hk, max_len, chunk):
     """One split per row for rows of at most 512 keys that give a workgroup per
-    CU (256), 128-key splits up to 512 workgroups (256 for MHA and beyond
-    eight splits), the long-launch rule past that."""
+    CU (256); 128-key splits where they take no more rounds of 256 workgroups than
+    256-key ones (one round for MHA and beyond eight splits) and up to 32 or 48
+    per row; the long-launch rule past that."""
     p = oa.decode_plan(rows, hq, hk, 16, max_len)
     assert p.chunk == chunk and p.splits == -(-max_len // chunk)
     assert p.workspace_bytes == (rows * hq * p.splits * 129 * 4 if p.splits > 1 else 0)
