@@ -331,7 +331,8 @@ int omni_hidream_qk_rope(void* qkv, int ld, const void* q_norm, const void* k_no
  * (tiles % resident workgroups, if at most half a round) is split by keys into
  * chunks that fill the round, and a combine kernel merges the chunks
  * (log-sum-exp). A call of less than a round is split so only where at least
- * four chunks of four key tiles fit (few heads, many queries); else it runs as
+ * four (past a quarter of the GPU, three) chunks of four key tiles fit (few heads,
+ * many queries); else it runs as
  * omni_hidream_attend_batched. Same results to rounding (rows of split tiles
  * round with the split); workspace NULL runs as omni_hidream_attend_batched.
  * workspace_bytes must be at least omni_hidream_workspace_bytes() (16-byte

@@ -995,15 +995,18 @@ void dit_split(const TiledArgs& a, int batch, int resident, int* items, int* spl
   const int rem = (int)(n % resident);
   if (rem == 0 || resident / rem < 2) return;
   const int chunks = std::min(resident / rem, std::max(2, (a.q_len + kBN - 1) / kBN / kMinChunkTiles));
-  // Calls of less than one round that would get only two or three chunks run as
-  // row parts within the launch instead (tiled_quarters, dit_halves): no partials
-  // in memory and no combine launch. us per call, by keys / by rows, 32q/8kv:
+  // Calls of less than one round that would get only two chunks, or three where
+  // they can run as quarters, run as row parts within the launch instead
+  // (tiled_quarters, dit_halves): no partials in memory and no combine launch. us per call, by keys / by rows, 32q/8kv:
   // 65 queries x 142 keys 14.7 / 8.0, 257 x 334 20.6 / 10.0, 257 x 4096 53.9 / 52.6,
   // 1000 x 1077 37.3 / 23.5, 1024 x 4096 73.5 / 67.5 (past some 5000 keys for 257
   // queries and 9000 for 1024 two chunks win again: 257 x 8192 92 / 100; the host
-  // does not know the key count). Four chunks, 4q/1kv, 4000 x 4000: 45.9 / 54.4;
+  // does not know the key count; nor do quarters win for a handful of queries over
+  // as many keys: 25 x 4590 50 / 64, 26 x 4776 of 16q/8kv 51 / 67, but 65 x 142 as
+  // above). Three chunks: in quarters 8q/8kv 1709 x 1721 38 / 31, as halves 2280 x
+  // 2280 44.2 / 48.3, 8q/1kv 2621 x 2621 causal 44.8 / 52.3. Four chunks, 4q/1kv, 4000 x 4000: 45.9 / 54.4;
   // 8q/1kv, 2048 x 8192 72 / 103, 2048 x 2048 35.2 / 30.2.
-  if (n < resident && chunks < 4) return;
+  if (n < resident && chunks < (tiled_quarters(n, resident) ? 4 : 3)) return;
   *split_from = (int)n - rem;
   *split_k = chunks;
 }

@@ -119,7 +119,7 @@ def dit_path(hq, hk, q_len, batch=1, ws=False):
     rem = items % cus
     if ws and 0 < rem <= cus // 2:
         chunks = min(cus // rem, max(2, -(-q_len // 128) // 4))
-        if items >= cus or chunks >= 4:
+        if items >= cus or chunks >= (4 if items * 4 <= cus else 3):
             return f"{chunks} chunks"
     return "quarters" if items * 4 <= cus else "halves" if 0 < rem <= cus // 2 else "whole"
 
@@ -198,6 +198,7 @@ SPLITS = [
     (32, 4, 2060, 520, 1, 4),    # 260; 5 key tiles
     (32, 32, 257, 300, 5, 2),    # 320
     (8, 1, 1921, 1000, 1, 4),    # 61 tiles, all split
+    (8, 8, 2049, 600, 1, 3),     # 72, all split
 ]
 
 
@@ -492,8 +493,9 @@ def splits_by_keys(hq, hk, q_len, batch=1):
 
 
 @pytest.mark.parametrize("hq,hk,q_len,batch,split", [
-    # below one round (256 CUs): by rows, unless at least four chunks of four key tiles fit
+    # below one round (256 CUs): by rows, unless at least four chunks of four key tiles fit, three past 64 tiles
     (32, 8, 65, 1, False), (32, 8, 1000, 1, False), (8, 1, 1920, 1, False), (8, 1, 1921, 1, True), (4, 1, 4000, 1, True),
+    (8, 8, 1920, 1, False), (8, 8, 2049, 1, True), (8, 8, 2560, 1, True), (8, 8, 2561, 1, False),  # 64, 72, 80 tiles: three chunks; 88: two
     (8, 2, 4000, 1, False),  # 126 items: two chunks
     # past a round: the remainder, if at most half a round
     (32, 8, 1100, 2, True), (32, 8, 2049, 1, True), (32, 8, 3000, 1, True), (32, 8, 3100, 1, False),
